@@ -125,8 +125,7 @@ KERNEL_NAMES = ["spmv", "mic_fwd", "mic_bwd", "pcg_update", "mic_factor", "p2g",
 # HIP kernel symbols behind each class (for matching rocprofv3 traces)
 KERNEL_SYMBOLS = {
     "spmv": ["k_spmv", "k_mg_spmv"], "mic_fwd": ["k_fwd"], "mic_bwd": ["k_bwd"], "pcg_update": ["k_update", "k_mg_update"],
-    "mic_factor": ["k_factor_sweep"], "p2g": ["k_p2g_records", "k_p2g_gather", "k_keys_nearest", "k_count",
-                                             "k_scatter", "k_sort_bins"],
+    "mic_factor": ["k_factor_sweep"], "p2g": ["k_p2g_records", "k_p2g_gather", "k_bin_count", "k_scatter"],
     "g2p": ["k_g2p"], "advect": ["k_advect"], "reconstruct": ["k_keys_morton", "k_bin_last", "k_recon_splat",
                                                                "k_recon_final"],
     "mg_level0": ["k_mg_pre", "k_mg_restrict", "k_mg_post1", "k_mg_post2"], "mg_coarse": [],

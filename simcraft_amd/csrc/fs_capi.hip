@@ -93,7 +93,7 @@ void release_all(fs_ctx* c) {
   for (DBuf* b : {&c->surf_v, &c->surf_n, &c->surf_i, &c->apicc}) fs_free(*b);
   for (DBuf* b : {&c->fsdf, &c->fsdfbuf, &c->sdfvalid, &c->sdfvalidbuf, &c->collider, &c->pg, &c->adiag, &c->rhs,
                   &c->active, &c->keys, &c->slots, &c->perm, &c->counts, &c->offs, &c->scan_tmp, &c->red,
-                  &c->recon_tmp, &c->sorted[0], &c->sorted[1], &c->sorted[2], &c->sorted[3], &c->p2g_w,
+                  &c->recon_tmp, &c->sorted[0], &c->sorted[1], &c->p2g_w,
                   &c->p2g_tiles, &c->offs2, &c->p2g_w2, &c->p2g_tiles2, &c->rkeys, &c->rbinmax, &c->rbins})
     fs_free(*b);
   for (int q = 0; q < 6; q++) fs_free(c->an[q]);
@@ -373,7 +373,7 @@ int fs_set_particles(fs_ctx* c, const double* pos, const double* vel, int64_t n)
     fs_free(c->keys);
     fs_free(c->slots);
     fs_free(c->perm);
-    for (int q = 0; q < 4; q++) fs_free(c->sorted[q]);
+    for (int q = 0; q < 2; q++) fs_free(c->sorted[q]);
     fs_free(c->p2g_w);
     fs_free(c->p2g_w2);
     fs_free(c->rkeys);
@@ -383,12 +383,18 @@ int fs_set_particles(fs_ctx* c, const double* pos, const double* vel, int64_t n)
       FS_TRY(fs_alloc(c, c->vel[d], (size_t)n * c->rsz));
     }
     FS_TRY(fs_alloc(c, c->staging, (size_t)n * 3 * sizeof(double)));
-    FS_TRY(fs_alloc(c, c->keys, (size_t)n * sizeof(int)));
-    FS_TRY(fs_alloc(c, c->slots, (size_t)n * sizeof(int)));
-    FS_TRY(fs_alloc(c, c->perm, (size_t)n * sizeof(int)));
-    for (int q = 0; q < 4; q++) FS_TRY(fs_alloc(c, c->sorted[q], (size_t)n * c->rsz));
-    FS_TRY(fs_alloc(c, c->p2g_w, (size_t)n * 12 * c->rsz));
-    FS_TRY(fs_alloc(c, c->p2g_w2, (size_t)n * 12 * c->rsz));
+    // P2G: one buffer set for the three face grids together, or two sets of one face grid each
+    const bool batch = fs_p2g_batch(n);
+    const size_t nr = (size_t)n * (batch ? 3 : 1);
+    FS_TRY(fs_alloc(c, c->keys, nr * sizeof(int)));
+    FS_TRY(fs_alloc(c, c->slots, nr * sizeof(int)));
+    FS_TRY(fs_alloc(c, c->perm, nr * sizeof(int)));
+    FS_TRY(fs_alloc(c, c->sorted[0], nr * c->rsz));
+    FS_TRY(fs_alloc(c, c->p2g_w, nr * 12 * c->rsz));
+    if (!batch) {
+      FS_TRY(fs_alloc(c, c->sorted[1], nr * c->rsz));
+      FS_TRY(fs_alloc(c, c->p2g_w2, nr * 12 * c->rsz));
+    }
     FS_TRY(fs_alloc(c, c->rkeys, (size_t)n * sizeof(int)));
     c->np = n;
   }

@@ -158,10 +158,10 @@ struct fs_ctx {
   DBuf adiag, an[6], rhs, active;
   // binning
   DBuf keys, slots, perm, counts, offs, scan_tmp;
-  DBuf sorted[4];   // bin-ordered velocity component (P2G); spare particle-sized scratch
+  DBuf sorted[2];   // bin-ordered velocity component (P2G), one per buffer set
   DBuf p2g_w;       // 12 kernel factors per particle in bin order (P2G)
   DBuf recon_tmp;   // per-cell squared-distance minima, one array per XCD and a spare (reconstruction)
-  DBuf p2g_tiles;   // P2G gather tile keys and heaviest-first tile order
+  DBuf p2g_tiles;   // P2G gather tile work and heaviest-first tile order
   // second P2G buffer set (bin offsets, records, tile order; the velocity records go to
   // sorted[1]): a face grid's gather runs on `side` while the next face grid is binned
   DBuf offs2, p2g_w2, p2g_tiles2;
@@ -260,6 +260,9 @@ int fs_particles_download(fs_ctx* c, double* pos, double* vel);
 // Conversions between the FP64 ABI and device storage of a given real size.
 int fs_upload_real(fs_ctx* c, DBuf& dst, const double* src, size_t n);
 int fs_download_real(fs_ctx* c, const DBuf& src, double* dst, size_t n);
+
+// Up to this many particles P2G bins and gathers the three face grids together.
+inline bool fs_p2g_batch(int64_t n) { return n <= (int64_t)1 << 22; }
 
 inline unsigned fs_blocks(int64_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }
 
