@@ -42,7 +42,12 @@ namespace {
 
 constexpr double MG_OMEGA = 0.9;  // Jacobi weight
 constexpr double MG_ALPHA = 1.8;  // coarse-correction weight
-constexpr int MCH = 4096;         // cells per block
+constexpr int MCH = 4096;         // cells per block of the kernels that reduce
+// Up to this many blocks of them take 1024 threads instead of 256 (chunk_sum): with few blocks a
+// thread's sixteen cells in turn are the kernel's time, with many the other blocks hide them. Mixed,
+// us, 256 / 1024 threads, SpMV, last sweep, update: 128^3 38.5 / 15.9, 21.8 / 9.8, 13.4 / 9.0; 192^3
+// (1728 blocks) 52.7 / 34.5, 28.5 / 20.2, 22.2 / 22.4; 256^3 (4096) 75 / 78, 38.4 / 44.2, 41.3 / 50.7.
+constexpr unsigned MG_WIDE = 2048;
 
 template <typename S>
 struct Lv {
@@ -80,9 +85,12 @@ __global__ __launch_bounds__(256) void k_mg_level0(int nx, int ny, int nz, const
                                                    const S* __restrict__ aL, const S* __restrict__ aD,
                                                    const S* __restrict__ aB, const uint8_t* __restrict__ act,
                                                    S* __restrict__ D, S* __restrict__ Cx, S* __restrict__ Cy,
-                                                   S* __restrict__ Cz, S* __restrict__ W) {
+                                                   S* __restrict__ Cz, S* __restrict__ W, S* __restrict__ x,
+                                                   S* __restrict__ xs) {
   const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (c >= (int64_t)nx * ny * nz) return;
+  x[c] = S(0);  // the cycle never writes a cell with W = 0: its iterates stay 0 for the solve
+  xs[c] = S(0);
   int i, j, k;
   decode3(c, ny, nz, i, j, k);
   const int64_t sx = (int64_t)ny * nz;
@@ -104,9 +112,11 @@ __global__ __launch_bounds__(256) void k_mg_level0(int nx, int ny, int nz, const
 template <typename S>
 __global__ __launch_bounds__(256) void k_mg_coarsen(Lv<S> F, int cx_, int cy_, int cz_, S* __restrict__ D,
                                                     S* __restrict__ Cx, S* __restrict__ Cy, S* __restrict__ Cz,
-                                                    S* __restrict__ W) {
+                                                    S* __restrict__ W, S* __restrict__ x, S* __restrict__ xs) {
   const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (c >= (int64_t)cx_ * cy_ * cz_) return;
+  x[c] = S(0);
+  xs[c] = S(0);
   int I, J, K;
   decode3(c, cy_, cz_, I, J, K);
   S d = S(0), sx = S(0), sy = S(0), sz = S(0);
@@ -143,20 +153,24 @@ __device__ __forceinline__ S pre_cell(const Lv<S>& L, const B* __restrict__ b, i
   auto xo = [&](int64_t q, int, int, int) { return L.W[q] * (S)b[q]; };
   return xo(c, i, j, k) + L.W[c] * ((S)b[c] - row<S>(L, c, i, j, k, xo));
 }
-// b(f) - (A x)(f) summed over the live children f of aggregate (I, J, K), in lexicographic order.
+// b(f) - (A x)(f) of child (bits di dj dk of q) of aggregate (I, J, K), 0 when it is off the grid or
+// not live (adding it then changes no bit of the aggregate's sum, which starts at +0).
 template <typename S, typename B>
-__device__ __forceinline__ S restrict_cell(const Lv<S>& L, const B* __restrict__ b, const S* __restrict__ x, int I,
-                                           int J, int K) {
-  auto xo = [&](int64_t q, int, int, int) { return x[q]; };
+__device__ __forceinline__ S restrict_child(const Lv<S>& L, const B* __restrict__ b, const S* __restrict__ x, int I,
+                                            int J, int K, int q) {
+  auto xo = [&](int64_t c, int, int, int) { return x[c]; };
+  const int i = 2 * I + (q >> 2), j = 2 * J + ((q >> 1) & 1), k = 2 * K + (q & 1);
+  if (i >= L.nx || j >= L.ny || k >= L.nz) return S(0);
+  const int64_t f = ((int64_t)i * L.ny + j) * L.nz + k;
+  return L.W[f] > S(0) ? (S)b[f] - row<S>(L, f, i, j, k, xo) : S(0);
+}
+// Sum over the children of an aggregate, which are eight consecutive lanes, in lexicographic order.
+template <typename S>
+__device__ __forceinline__ S restrict_sum(S r) {
+  const int l0 = threadIdx.x & 56;
   S acc = S(0);
-  for (int di = 0; di < 2; di++)
-    for (int dj = 0; dj < 2; dj++)
-      for (int dk = 0; dk < 2; dk++) {
-        const int i = 2 * I + di, j = 2 * J + dj, k = 2 * K + dk;
-        if (i >= L.nx || j >= L.ny || k >= L.nz) continue;
-        const int64_t f = ((int64_t)i * L.ny + j) * L.nz + k;
-        if (L.W[f] > S(0)) acc = acc + ((S)b[f] - row<S>(L, f, i, j, k, xo));
-      }
+#pragma unroll
+  for (int q = 0; q < 8; q++) acc = acc + __shfl(r, l0 + q, 64);
   return acc;
 }
 // The coarse correction x' = x + alpha xc(parent) on live cells, then one sweep at a live cell.
@@ -191,16 +205,30 @@ __global__ __launch_bounds__(256) void k_mg_pre(Lv<S> L, const B* __restrict__ b
   x[c] = pre_cell<S, B>(L, b, c, i, j, k);
 }
 
-template <typename S, typename B>
+// CHILD: one thread per child, the aggregate's sum over eight lanes; else one thread per aggregate.
+// Eight residuals of seven operands each, one after another in a thread, are the slowest sweep of a
+// small level (mixed, us, an aggregate / a child per thread: 7.2 / 3.3 for 64^3 -> 32^3, 11.0 / 10.0
+// for 128^3); above, other waves hide them and the eightfold threads and their shuffles cost more
+// than they save (14.8 / 17.0 for 160^3, 39.8 / 54.5 for 256^3).
+constexpr int64_t MG_RESTRICT_CHILD = (int64_t)1 << 18;  // aggregates up to which CHILD is taken
+template <typename S, typename B, bool CHILD>
 __global__ __launch_bounds__(256) void k_mg_restrict(Lv<S> L, const B* __restrict__ b, const S* __restrict__ x,
                                                      int cnx, int cny, int cnz, S* __restrict__ bc,
                                                      const PcgScalars* sc) {
   if (sc && sc->converged != STOP_RUN) return;
-  const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (c >= (int64_t)cnx * cny * cnz) return;
+  const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, c = CHILD ? e >> 3 : e;
+  if (c >= (int64_t)cnx * cny * cnz) return;  // uniform over the eight lanes of an aggregate
   int I, J, K;
   decode3(c, cny, cnz, I, J, K);
-  bc[c] = restrict_cell<S, B>(L, b, x, I, J, K);
+  if constexpr (CHILD) {
+    const int q = threadIdx.x & 7;
+    const S acc = restrict_sum<S>(restrict_child<S, B>(L, b, x, I, J, K, q));
+    if (q == 0) bc[c] = acc;
+  } else {
+    S acc = S(0);
+    for (int q = 0; q < 8; q++) acc = acc + restrict_child<S, B>(L, b, x, I, J, K, q);
+    bc[c] = acc;
+  }
 }
 
 template <typename S, typename B>
@@ -230,26 +258,23 @@ __global__ __launch_bounds__(256) void k_mg_sweep(Lv<S> L, const B* __restrict__
 // The sweep that ends a CG cycle on level 0, from xs into x = z, with z.r over the chunk, reduced by
 // the last block into sigma (FIRST: the initial sigma; else beta = sigma_new / sigma,
 // sigma = sigma_new). Chunks of 4096 cells per block: the fixed reduction tree.
-template <typename S, typename B, bool DOT, bool FIRST>
-__global__ __launch_bounds__(256) void k_mg_post2(Lv<S> L, const B* __restrict__ b, const S* __restrict__ xs,
+template <typename S, typename B, bool FIRST, int TH>
+__global__ __launch_bounds__(TH) void k_mg_post2(Lv<S> L, const B* __restrict__ b, const S* __restrict__ xs,
                                                   S* __restrict__ x, double* __restrict__ part, int nchunks,
                                                   PcgScalars* sc) {
   __shared__ double sm[4];
   if (sc && sc->converged != STOP_RUN) return;
+  __shared__ double terms[CHUNK_TERMS<TH>];
   const int64_t n = (int64_t)L.nx * L.ny * L.nz;
-  double acc = 0.0;
-#pragma unroll 1
-  for (int m = 0; m < 16; m++) {
-    const int64_t c = (int64_t)blockIdx.x * MCH + m * 256 + threadIdx.x;
-    if (c >= n) break;
-    if (!(L.W[c] > S(0))) continue;  // z = 0 there, and so is its product with r
+  const double acc = chunk_sum<TH>(terms, [&](int e) __attribute__((always_inline)) {
+    const int64_t c = (int64_t)blockIdx.x * MCH + e;
+    if (c >= n || !(L.W[c] > S(0))) return 0.0;  // z = 0 there, and so is its product with r
     int i, j, k;
     decode3(c, L.ny, L.nz, i, j, k);
     const S out = sweep_cell<S, B>(L, b, xs, c, i, j, k);
     x[c] = out;
-    if (DOT) acc += (double)out * (double)b[c];
-  }
-  if (!DOT) return;
+    return (double)out * (double)b[c];
+  });
   const double bs = block_sum256(acc, sm);
   if (threadIdx.x == 0) xstore(part + blockIdx.x, bs);
   if (blockIdx.x == gridDim.x - 1) {
@@ -264,67 +289,107 @@ __global__ __launch_bounds__(256) void k_mg_post2(Lv<S> L, const B* __restrict__
 
 // The levels from l0 down to the single cell and back up, in one workgroup (the small levels,
 // where separate launches would cost more than the work): the same cell functions, the passes
-// separated by workgroup barriers.
+// separated by workgroup barriers. The iterates and right-hand sides of all its levels live in
+// LDS, as do the operators in FP32 (in FP64 the first level's operator, 160 KB, stays in memory):
+// a pass is then a few LDS reads instead of dependent reads of the L2 (19 passes at 64^3:
+// 29.5 -> 15.1 us in FP32).
 constexpr int MG_TAIL_CELLS = 4096;  // levels at or below this size run in the tail kernel
+constexpr int MG_TAIL_SUM = 4800;    // ... if all its levels together have no more cells than this
 constexpr int MG_MAX_LEVELS = 16;
 template <typename S>
 struct TailLevels {
   Lv<S> L[MG_MAX_LEVELS];
-  S* b[MG_MAX_LEVELS];
-  S* x[MG_MAX_LEVELS];
-  S* xs[MG_MAX_LEVELS];
+  int off[MG_MAX_LEVELS + 1];  // of a level's cells in the tail's LDS arrays
+  const S* b;                  // right-hand side of level l0
+  S* x;                        // its solution
 };
 template <typename S>
 __global__ __launch_bounds__(1024) void k_mg_tail(TailLevels<S> T, int l0, int nl, S alpha, const PcgScalars* sc) {
+  constexpr bool ALL = sizeof(S) == 4;                    // level l0's operator in LDS as well
+  constexpr int CSUM = ALL ? MG_TAIL_SUM : MG_TAIL_SUM - MG_TAIL_CELLS;
+  __shared__ S cD[CSUM], cX[CSUM], cY[CSUM], cZ[CSUM], cW[CSUM], vb[MG_TAIL_SUM], vx[MG_TAIL_SUM], vs[MG_TAIL_SUM];
   if (sc && sc->converged != STOP_RUN) return;
   const int tid = threadIdx.x;
-  for (int l = l0; l < nl; l++) {
-    const Lv<S>& L = T.L[l];
-    const int n = L.nx * L.ny * L.nz;
+  const int n0 = T.off[l0 + 1];  // cells of level l0
+  const int c0 = ALL ? 0 : n0;   // the first cell whose operator is in LDS
+  for (int c = tid; c < T.off[nl]; c += 1024) {
+    vx[c] = S(0);  // cells with W = 0 are never written
+    vs[c] = S(0);
+    vb[c] = c < n0 ? T.b[c] : S(0);
+  }
+  for (int l = ALL ? l0 : l0 + 1; l < nl; l++) {
+    const int n = T.off[l + 1] - T.off[l], o = T.off[l] - c0;
+    for (int c = tid; c < n; c += 1024) {
+      cD[o + c] = T.L[l].D[c];
+      cX[o + c] = T.L[l].Cx[c];
+      cY[o + c] = T.L[l].Cy[c];
+      cZ[o + c] = T.L[l].Cz[c];
+      cW[o + c] = T.L[l].W[c];
+    }
+  }
+  __syncthreads();
+  auto in_lds = [&](int l) {
+    const int o = T.off[l] - c0;
+    return Lv<S>{T.L[l].nx, T.L[l].ny, T.L[l].nz, cD + o, cX + o, cY + o, cZ + o, cW + o};
+  };
+  auto down = [&](int l, const Lv<S>& L) __attribute__((always_inline)) {
+    const int n = L.nx * L.ny * L.nz, o = T.off[l];
     for (int c = tid; c < n; c += 1024) {
       if (!(L.W[c] > S(0))) continue;
       int i, j, k;
       decode3(c, L.ny, L.nz, i, j, k);
-      T.x[l][c] = pre_cell<S, S>(L, T.b[l], c, i, j, k);
+      vx[o + c] = pre_cell<S, S>(L, vb + o, c, i, j, k);
     }
     __syncthreads();
     if (l + 1 < nl) {
-      const Lv<S>& C = T.L[l + 1];
-      const int nc = C.nx * C.ny * C.nz;
-      for (int c = tid; c < nc; c += 1024) {
+      const int cny = T.L[l + 1].ny, cnz = T.L[l + 1].nz, on = T.off[l + 1], nc = T.off[l + 2] - on;
+      for (int e = tid; e < 8 * nc; e += 1024) {
         int I, J, K;
-        decode3(c, C.ny, C.nz, I, J, K);
-        T.b[l + 1][c] = restrict_cell<S, S>(L, T.b[l], T.x[l], I, J, K);
+        decode3(e >> 3, cny, cnz, I, J, K);
+        const S acc = restrict_sum<S>(restrict_child<S, S>(L, vb + o, vx + o, I, J, K, e & 7));
+        if ((e & 7) == 0) vb[on + (e >> 3)] = acc;
       }
       __syncthreads();
     }
-  }
-  auto sweep = [&](int l, const S* from, S* to) {
-    const Lv<S>& L = T.L[l];
-    const int n = L.nx * L.ny * L.nz;
+  };
+  auto sweep = [&](int l, const Lv<S>& L, const S* from, S* to) __attribute__((always_inline)) {
+    const int n = L.nx * L.ny * L.nz, o = T.off[l];
     for (int c = tid; c < n; c += 1024) {
       if (!(L.W[c] > S(0))) continue;
       int i, j, k;
       decode3(c, L.ny, L.nz, i, j, k);
-      to[c] = sweep_cell<S, S>(L, T.b[l], from, c, i, j, k);
+      to[o + c] = sweep_cell<S, S>(L, vb + o, from + o, c, i, j, k);
     }
     __syncthreads();
   };
-  sweep(nl - 1, T.x[nl - 1], T.xs[nl - 1]);
-  sweep(nl - 1, T.xs[nl - 1], T.x[nl - 1]);
-  for (int l = nl - 2; l >= l0; l--) {
-    const Lv<S>& L = T.L[l];
-    const Lv<S>& C = T.L[l + 1];
-    const int n = L.nx * L.ny * L.nz;
+  auto up = [&](int l, const Lv<S>& L) __attribute__((always_inline)) {
+    const int cny = T.L[l + 1].ny, cnz = T.L[l + 1].nz, on = T.off[l + 1];
+    const int n = L.nx * L.ny * L.nz, o = T.off[l];
     for (int c = tid; c < n; c += 1024) {
       if (!(L.W[c] > S(0))) continue;
       int i, j, k;
       decode3(c, L.ny, L.nz, i, j, k);
-      T.xs[l][c] = post1_cell<S, S>(L, T.b[l], T.x[l], T.x[l + 1], C.ny, C.nz, alpha, c, i, j, k);
+      vs[o + c] = post1_cell<S, S>(L, vb + o, vx + o, vx + on, cny, cnz, alpha, c, i, j, k);
     }
     __syncthreads();
-    sweep(l, T.xs[l], T.x[l]);
+    sweep(l, L, vs, vx);
+  };
+  if (ALL) down(l0, in_lds(l0));
+  else down(l0, T.L[l0]);
+  for (int l = l0 + 1; l < nl; l++) down(l, in_lds(l));
+  if (ALL || nl - 1 > l0) {
+    sweep(nl - 1, in_lds(nl - 1), vx, vs);
+    sweep(nl - 1, in_lds(nl - 1), vs, vx);
+  } else {
+    sweep(l0, T.L[l0], vx, vs);
+    sweep(l0, T.L[l0], vs, vx);
   }
+  for (int l = nl - 2; l > l0; l--) up(l, in_lds(l));
+  if (nl - 1 > l0) {
+    if (ALL) up(l0, in_lds(l0));
+    else up(l0, T.L[l0]);
+  }
+  for (int c = tid; c < n0; c += 1024) T.x[c] = vx[c];
 }
 
 // ---- CG kernels ---------------------------------------------------------------------------------
@@ -333,7 +398,9 @@ __global__ __launch_bounds__(1024) void k_mg_tail(TailLevels<S> T, int l0, int n
 template <typename T>
 __global__ __launch_bounds__(256) void k_mg_init(int64_t n, const uint8_t* __restrict__ act,
                                                  const T* __restrict__ rhs, double* __restrict__ x,
-                                                 double* __restrict__ r, double* __restrict__ part,
+                                                 double* __restrict__ r, double* __restrict__ s0,
+                                                 double* __restrict__ s1, double* __restrict__ t,
+                                                 double* __restrict__ part,
                                                  double* __restrict__ part2, int nchunks, PcgScalars* sc,
                                                  int tol_mode, double tol) {
   __shared__ double sm[4];
@@ -345,6 +412,9 @@ __global__ __launch_bounds__(256) void k_mg_init(int64_t n, const uint8_t* __res
     const double v = act[c] ? (double)rhs[c] : 0.0;
     r[c] = v;
     x[c] = 0.0;
+    s0[c] = 0.0;  // s and t are written on active cells only
+    s1[c] = 0.0;
+    t[c] = 0.0;
     ss += v * v;
     const double av = act[c] ? fabs(v) : 0.0;
     mx = (mx < av) ? av : mx;
@@ -379,8 +449,8 @@ __global__ __launch_bounds__(256) void k_mg_init(int64_t n, const uint8_t* __res
 // s = z (iteration 1) or z + beta s_old, recomputed for the six neighbours; t = A s (the assembled
 // system in FP64 on active cells); s.t reduced by the last block into alpha. Inactive cells are not
 // written: s and t are zeroed when the solve starts and stay 0 there.
-template <typename S>
-__global__ __launch_bounds__(256) void k_mg_spmv(Lv<S> L, const uint8_t* __restrict__ act, const S* __restrict__ z,
+template <typename S, int TH>
+__global__ __launch_bounds__(TH) void k_mg_spmv(Lv<S> L, const uint8_t* __restrict__ act, const S* __restrict__ z,
                                                  const double* __restrict__ s_old, double* __restrict__ s_new,
                                                  double* __restrict__ t, double* __restrict__ part, int nchunks,
                                                  PcgScalars* sc, int iter) {
@@ -390,20 +460,18 @@ __global__ __launch_bounds__(256) void k_mg_spmv(Lv<S> L, const uint8_t* __restr
   const bool first = iter == 1;
   const double beta = sc->beta;
   auto so = [&](int64_t q, int, int, int) { return first ? (double)z[q] : (double)z[q] + beta * s_old[q]; };
-  double acc = 0.0;
-#pragma unroll 1
-  for (int m = 0; m < 16; m++) {
-    const int64_t c = (int64_t)blockIdx.x * MCH + m * 256 + threadIdx.x;
-    if (c >= n) break;
-    if (!act[c]) continue;
+  __shared__ double terms[CHUNK_TERMS<TH>];
+  const double acc = chunk_sum<TH>(terms, [&](int e) __attribute__((always_inline)) {
+    const int64_t c = (int64_t)blockIdx.x * MCH + e;
+    if (c >= n || !act[c]) return 0.0;
     int i, j, k;
     decode3(c, L.ny, L.nz, i, j, k);
     const double sv = so(c, i, j, k);
     const double tv = row<double>(L, c, i, j, k, so);
     s_new[c] = sv;
     t[c] = tv;
-    acc += sv * tv;
-  }
+    return sv * tv;
+  });
   const double bs = block_sum256(acc, sm);
   if (threadIdx.x == 0) xstore(part + blockIdx.x, bs);
   if (blockIdx.x == gridDim.x - 1) {
@@ -424,7 +492,8 @@ __global__ __launch_bounds__(256) void k_mg_spmv(Lv<S> L, const uint8_t* __restr
 
 // x += alpha s, r += -alpha t on active cells (saxpy, util.cc:394-402); ||r||_inf, ||r||_2^2 and the
 // stopping test of iteration iter.
-__global__ __launch_bounds__(256) void k_mg_update(int64_t n, const uint8_t* __restrict__ act,
+template <int TH>
+__global__ __launch_bounds__(TH) void k_mg_update(int64_t n, const uint8_t* __restrict__ act,
                                                    double* __restrict__ x, const double* __restrict__ s,
                                                    double* __restrict__ r, const double* __restrict__ t,
                                                    double* __restrict__ part, double* __restrict__ part2,
@@ -432,18 +501,19 @@ __global__ __launch_bounds__(256) void k_mg_update(int64_t n, const uint8_t* __r
   __shared__ double sm[4];
   if (sc->converged != STOP_RUN) return;
   const double alpha = sc->alpha;
-  double mx = 0.0, ss = 0.0;
-  for (int m = 0; m < 16; m++) {
-    const int64_t c = (int64_t)blockIdx.x * MCH + m * 256 + threadIdx.x;
-    if (c >= n) break;
-    if (!act[c]) continue;  // r = 0 there
+  __shared__ double terms[CHUNK_TERMS<TH>];
+  double mx = 0.0;
+  const double ss = chunk_sum<TH>(terms, [&](int e) __attribute__((always_inline)) {
+    const int64_t c = (int64_t)blockIdx.x * MCH + e;
+    if (c >= n || !act[c]) return 0.0;  // r = 0 there
     x[c] = x[c] + alpha * s[c];
     const double rv = r[c] + (-alpha) * t[c];
     r[c] = rv;
     const double av = fabs(rv);
     mx = (mx < av) ? av : mx;
-    ss += rv * rv;
-  }
+    return rv * rv;
+  });
+  mx = chunk_max<TH>(mx, terms);
   const double bm = block_max256(mx, sm);
   const double bs = block_sum256(ss, sm);
   if (threadIdx.x == 0) {
@@ -510,9 +580,6 @@ int mg_build(fs_ctx* c) {
     const size_t bytes = (size_t)B.n * sizeof(S);
     for (DBuf* d : {&B.D, &B.Cx, &B.Cy, &B.Cz, &B.W, &B.x, &B.xs}) FS_TRY(ensure(c, *d, bytes));
     if (l > 0) FS_TRY(ensure(c, B.b, bytes));
-    // the cycle never writes a cell with W = 0: its iterates stay 0 there for the solve
-    FS_HIP(c, hipMemsetAsync(B.x.p, 0, bytes, c->stream));
-    FS_HIP(c, hipMemsetAsync(B.xs.p, 0, bytes, c->stream));
   }
   if ((int)M.lv.size() > MG_MAX_LEVELS) {
     c->set_error("multigrid: too many levels");
@@ -521,12 +588,14 @@ int mg_build(fs_ctx* c) {
   MgLevelBuf& L0 = M.lv[0];
   k_mg_level0<S><<<fs_blocks(L0.n, 256), 256, 0, c->stream>>>(
       c->nx, c->ny, c->nz, c->adiag.as<S>(), c->an[0].as<S>(), c->an[3].as<S>(), c->an[5].as<S>(),
-      c->active.as<uint8_t>(), L0.D.as<S>(), L0.Cx.as<S>(), L0.Cy.as<S>(), L0.Cz.as<S>(), L0.W.as<S>());
+      c->active.as<uint8_t>(), L0.D.as<S>(), L0.Cx.as<S>(), L0.Cy.as<S>(), L0.Cz.as<S>(), L0.W.as<S>(),
+      L0.x.as<S>(), L0.xs.as<S>());
   for (size_t l = 1; l < M.lv.size(); l++) {
     MgLevelBuf& B = M.lv[l];
     k_mg_coarsen<S><<<fs_blocks(B.n, 256), 256, 0, c->stream>>>(lv_of<S>(M.lv[l - 1]), B.nx, B.ny, B.nz,
                                                                   B.D.as<S>(), B.Cx.as<S>(), B.Cy.as<S>(),
-                                                                  B.Cz.as<S>(), B.W.as<S>());
+                                                                  B.Cz.as<S>(), B.W.as<S>(), B.x.as<S>(),
+                                                                  B.xs.as<S>());
   }
   FS_HIP(c, hipGetLastError());
   return FS_OK;
@@ -546,12 +615,15 @@ int mg_cycle(fs_ctx* c, const double* r0, PcgScalars* sc, bool first) {
   };
   auto restrict_ = [&](int l) {
     MgLevelBuf &B = M.lv[l], &C = M.lv[l + 1];
-    if (l == 0)
-      k_mg_restrict<S, double><<<fs_blocks(C.n, 256), 256, 0, c->stream>>>(lv_of<S>(B), r0, B.x.as<S>(), C.nx, C.ny,
-                                                                           C.nz, C.b.as<S>(), sc);
-    else
-      k_mg_restrict<S, S><<<fs_blocks(C.n, 256), 256, 0, c->stream>>>(lv_of<S>(B), B.b.as<S>(), B.x.as<S>(), C.nx,
-                                                                      C.ny, C.nz, C.b.as<S>(), sc);
+    auto go = [&](auto kern, const auto* b, int64_t threads) {
+      kern<<<fs_blocks(threads, 256), 256, 0, c->stream>>>(lv_of<S>(B), b, B.x.as<S>(), C.nx, C.ny, C.nz, C.b.as<S>(),
+                                                           sc);
+    };
+    const bool child = C.n <= MG_RESTRICT_CHILD;
+    if (l == 0 && child) go(k_mg_restrict<S, double, true>, r0, 8 * C.n);
+    else if (l == 0) go(k_mg_restrict<S, double, false>, r0, C.n);
+    else if (child) go(k_mg_restrict<S, S, true>, (const S*)B.b.as<S>(), 8 * C.n);
+    else go(k_mg_restrict<S, S, false>, (const S*)B.b.as<S>(), C.n);
   };
   auto post1 = [&](int l) {
     MgLevelBuf &B = M.lv[l], &C = M.lv[l + 1];
@@ -574,22 +646,25 @@ int mg_cycle(fs_ctx* c, const double* r0, PcgScalars* sc, bool first) {
       k_mg_sweep<S, S><<<nc1, 256, 0, c->stream>>>(L, B.b.as<S>(), from.as<S>(), to.as<S>(), sc);
     } else if (!last || !sc) {
       k_mg_sweep<S, double><<<nc1, 256, 0, c->stream>>>(L, r0, from.as<S>(), to.as<S>(), sc);
-    } else if (first) {
-      k_mg_post2<S, double, true, true><<<nb, 256, 0, c->stream>>>(L, r0, from.as<S>(), to.as<S>(),
-                                                                    M.partials.as<double>(), (int)nb, sc);
     } else {
-      k_mg_post2<S, double, true, false><<<nb, 256, 0, c->stream>>>(L, r0, from.as<S>(), to.as<S>(),
-                                                                     M.partials.as<double>(), (int)nb, sc);
+      auto go = [&](auto kern, int th) {
+        kern<<<nb, th, 0, c->stream>>>(L, r0, from.as<S>(), to.as<S>(), M.partials.as<double>(), (int)nb, sc);
+      };
+      const bool wide = nb <= MG_WIDE;
+      if (first && wide) go(k_mg_post2<S, double, true, 1024>, 1024);
+      else if (first) go(k_mg_post2<S, double, true, 256>, 256);
+      else if (wide) go(k_mg_post2<S, double, false, 1024>, 1024);
+      else go(k_mg_post2<S, double, false, 256>, 256);
     }
   };
-  // the levels from lt on run in one workgroup (the first level at or below MG_TAIL_CELLS cells,
-  // never level 0, whose right-hand side is the FP64 residual)
+  // the levels from lt on run in one workgroup (the first level small enough, with the levels
+  // below it, for the tail; never level 0, whose right-hand side is the FP64 residual)
   int lt = nl;
-  for (int l = 1; l < nl; l++)
-    if (M.lv[l].n <= MG_TAIL_CELLS) {
-      lt = l;
-      break;
-    }
+  for (int l = 1; l < nl && lt == nl; l++) {
+    int64_t sum = 0;
+    for (int m = l; m < nl; m++) sum += M.lv[m].n;
+    if (M.lv[l].n <= MG_TAIL_CELLS && sum <= MG_TAIL_SUM && sum - M.lv[l].n <= MG_TAIL_SUM - MG_TAIL_CELLS) lt = l;
+  }
   // down
   int pf = fs_prof_begin(c, FS_KERNEL_MG_LEVEL0, (16.0 + 12.0 * sizeof(S)) * na);
   pre(0);
@@ -604,12 +679,11 @@ int mg_cycle(fs_ctx* c, const double* r0, PcgScalars* sc, bool first) {
   if (lt < nl) {
     TailLevels<S> T{};
     for (int l = lt; l < nl; l++) {
-      MgLevelBuf& B = M.lv[l];
-      T.L[l] = lv_of<S>(B);
-      T.b[l] = B.b.as<S>();
-      T.x[l] = B.x.as<S>();
-      T.xs[l] = B.xs.as<S>();
+      T.L[l] = lv_of<S>(M.lv[l]);
+      T.off[l + 1] = T.off[l] + (int)M.lv[l].n;
     }
+    T.b = M.lv[lt].b.as<S>();
+    T.x = M.lv[lt].x.as<S>();
     k_mg_tail<S><<<1, 1024, 0, c->stream>>>(T, lt, nl, (S)MG_ALPHA, sc);
   }
   // up: correction and post-smoothing
@@ -673,9 +747,8 @@ int mg_solve_t(fs_ctx* c, fs_stats* st) {
   const double tol = c->cfg.cg_tolerance;
   const uint8_t* act = c->active.as<uint8_t>();
   FS_HIP(c, hipMemsetAsync(M.scal.p, 0, sizeof(PcgScalars), c->stream));
-  // s and t are written on active cells only
-  for (DBuf* d : {&M.s0, &M.s1, &M.t}) FS_HIP(c, hipMemsetAsync(d->p, 0, (size_t)n * sizeof(double), c->stream));
   k_mg_init<S><<<nb, 256, 0, c->stream>>>(n, act, c->rhs.as<S>(), M.x.as<double>(), M.r.as<double>(),
+                                           M.s0.as<double>(), M.s1.as<double>(), M.t.as<double>(),
                                            M.partials.as<double>(), M.partials2.as<double>(), nc, sc, tmode, tol);
   FS_HIP(c, hipGetLastError());
   FS_TRY(mg_read_scalars(c));
@@ -695,13 +768,20 @@ int mg_solve_t(fs_ctx* c, fs_stats* st) {
         const double* s_old = sb[(it + 1) & 1]->as<double>();
         double* s_new = sb[it & 1]->as<double>();
         int pf = fs_prof_begin(c, FS_KERNEL_SPMV, (24.0 + 5.0 * sizeof(S)) * c->n_active_last);
-        k_mg_spmv<S><<<nb, 256, 0, c->stream>>>(L, act, L0.x.as<S>(), s_old, s_new, M.t.as<double>(),
-                                                M.partials.as<double>(), nc, sc, it);
+        auto spmv = [&](auto kern, int th) {
+          kern<<<nb, th, 0, c->stream>>>(L, act, L0.x.as<S>(), s_old, s_new, M.t.as<double>(), M.partials.as<double>(),
+                                         nc, sc, it);
+        };
+        if (nb <= MG_WIDE) spmv(k_mg_spmv<S, 1024>, 1024);
+        else spmv(k_mg_spmv<S, 256>, 256);
         fs_prof_end(c, pf);
         pf = fs_prof_begin(c, FS_KERNEL_PCG_UPDATE, 48.0 * c->n_active_last);
-        k_mg_update<<<nb, 256, 0, c->stream>>>(n, act, M.x.as<double>(), s_new, M.r.as<double>(), M.t.as<double>(),
-                                              M.partials.as<double>(), M.partials2.as<double>(), nc, sc, it, tmode,
-                                              tol);
+        auto update = [&](auto kern, int th) {
+          kern<<<nb, th, 0, c->stream>>>(n, act, M.x.as<double>(), s_new, M.r.as<double>(), M.t.as<double>(),
+                                         M.partials.as<double>(), M.partials2.as<double>(), nc, sc, it, tmode, tol);
+        };
+        if (nb <= MG_WIDE) update(k_mg_update<1024>, 1024);
+        else update(k_mg_update<256>, 256);
         fs_prof_end(c, pf);
         FS_TRY(mg_cycle<S>(c, M.r.as<double>(), sc, false));
       }

@@ -23,12 +23,13 @@ __device__ inline double wave_max(double v) {
   }
   return v;
 }
-// 256-thread block: per-thread values -> (w0 + w1) + (w2 + w3) of wave butterflies.
+// Per-thread values of a block's first 256 threads -> (w0 + w1) + (w2 + w3) of wave butterflies
+// (the other threads of a larger block only take part in the barriers).
 __device__ inline double block_sum256(double v, double* sm) {
   double w = wave_sum(v);
   int wid = threadIdx.x >> 6;
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) sm[wid] = w;
+  if ((threadIdx.x & 63) == 0 && wid < 4) sm[wid] = w;
   __syncthreads();
   double r = (sm[0] + sm[1]) + (sm[2] + sm[3]);
   __syncthreads();
@@ -38,7 +39,7 @@ __device__ inline double block_max256(double v, double* sm) {
   double w = wave_max(v);
   int wid = threadIdx.x >> 6;
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) sm[wid] = w;
+  if ((threadIdx.x & 63) == 0 && wid < 4) sm[wid] = w;
   __syncthreads();
   double r = sm[0];
   for (int q = 1; q < 4; q++) r = (r < sm[q]) ? sm[q] : r;
@@ -110,12 +111,54 @@ __device__ __forceinline__ bool xunset(double v) { return (uint32_t)__double2hii
 // brick with the last ticket) waits until every entry is set, reduces them in the fixed order and
 // stores the sentinel back, so the entries are unset again for the next kernel.
 
-// Block-wide (256 threads) wait until p[0, n) are all set; false if the wait gave up.
+// Sum of the terms f(e), e = 0 .. 4095, of a chunk in the fixed order of 256 threads with 16 elements
+// each (thread t: e = t + 256 m, m ascending), by TH threads; the value is that of the first 256
+// threads. With TH = 1024, thread (g, t) = (tid / 256, tid % 256) evaluates m = 4g .. 4g + 3 and the
+// terms meet in LDS (TERMS<1024> doubles), so that a thread waits for four elements' loads in turn
+// instead of sixteen: the choice where a kernel has too few chunks to hide them by other blocks.
+template <int TH>
+constexpr int CHUNK_TERMS = TH == 256 ? 1 : 4096;
+template <int TH, class F>
+__device__ __forceinline__ double chunk_sum(double* terms, F&& f) {
+  double a = 0.0;
+  if constexpr (TH == 256) {
+#pragma unroll 1
+    for (int m = 0; m < 16; m++) a += f(256 * m + (int)threadIdx.x);
+  } else {
+    static_assert(TH == 1024, "four groups of 256 threads");
+    const int e0 = 1024 * (int)(threadIdx.x >> 8) + (int)(threadIdx.x & 255);
+#pragma unroll
+    for (int q = 0; q < 4; q++) terms[e0 + 256 * q] = f(e0 + 256 * q);
+    __syncthreads();
+    if (threadIdx.x < 256) {
+#pragma unroll
+      for (int m = 0; m < 16; m++) a += terms[256 * m + threadIdx.x];
+    }
+  }
+  return a;
+}
+// The maximum over a block's threads t, t + 256, .. to thread t of the first 256 (order-free).
+template <int TH>
+__device__ __forceinline__ double chunk_max(double mx, double* terms) {
+  if constexpr (TH > 256) {
+    __syncthreads();
+    terms[threadIdx.x] = mx;
+    __syncthreads();
+    if (threadIdx.x < 256)
+      for (int g = 1; g < TH / 256; g++) {
+        const double o = terms[256 * g + threadIdx.x];
+        mx = (mx < o) ? o : mx;
+      }
+  }
+  return mx;
+}
+
+// Block-wide wait until p[0, n) are all set; false if the wait gave up.
 __device__ inline bool gather_wait256(const double* p, int n, PcgScalars* sc) {
   long spins = 0;
   while (true) {
     int mine = 1;
-    for (int m = threadIdx.x; m < n; m += 256) mine &= xunset(xload(p + m)) ? 0 : 1;
+    for (int m = threadIdx.x; m < n; m += blockDim.x) mine &= xunset(xload(p + m)) ? 0 : 1;
     if (__syncthreads_and(mine)) return true;
     __builtin_amdgcn_s_sleep(2);
     int give = 0;
@@ -131,7 +174,7 @@ __device__ inline bool gather_wait256(const double* p, int n, PcgScalars* sc) {
 // block_sum256), which it returns to the sentinel.
 __device__ inline double gather_tree256(double* p, int n, double* sm) {
   double a = 0.0;
-  for (int m = threadIdx.x; m < n; m += 256) {
+  for (int m = threadIdx.x < 256 ? threadIdx.x : n; m < n; m += 256) {
     a += xload(p + m);
     xstore(p + m, xsent());
   }
@@ -140,7 +183,7 @@ __device__ inline double gather_tree256(double* p, int n, double* sm) {
 // max over gathered entries (order-free: the comparison never takes a NaN), returned to the sentinel
 __device__ inline double gather_max256(double* p, int n, double* sm) {
   double mx = 0.0;
-  for (int m = threadIdx.x; m < n; m += 256) {
+  for (int m = threadIdx.x < 256 ? threadIdx.x : n; m < n; m += 256) {
     const double v = xload(p + m);
     mx = (mx < v) ? v : mx;
     xstore(p + m, xsent());
