@@ -369,34 +369,23 @@ __global__ __launch_bounds__(TPB) void k_add(int64_t n, const T* __restrict__ a,
   if (id < n) b[id] = b[id] + a[id];
 }
 template <typename T>
-__global__ __launch_bounds__(TPB) void k_split3(int64_t n, const double* __restrict__ aos, T* __restrict__ x, T* __restrict__ y,
+__global__ __launch_bounds__(TPB) void k_split3(int64_t n, const T* __restrict__ aos, T* __restrict__ x, T* __restrict__ y,
                          T* __restrict__ z) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= n) return;
-  x[i] = (T)aos[3 * i];
-  y[i] = (T)aos[3 * i + 1];
-  z[i] = (T)aos[3 * i + 2];
+  x[i] = aos[3 * i];
+  y[i] = aos[3 * i + 1];
+  z[i] = aos[3 * i + 2];
 }
 template <typename T>
 __global__ __launch_bounds__(TPB) void k_join3(int64_t n, const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z,
-                        double* __restrict__ aos) {
+                        T* __restrict__ aos) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= n) return;
-  aos[3 * i] = (double)x[i];
-  aos[3 * i + 1] = (double)y[i];
-  aos[3 * i + 2] = (double)z[i];
+  aos[3 * i] = x[i];
+  aos[3 * i + 1] = y[i];
+  aos[3 * i + 2] = z[i];
 }
-template <typename T>
-__global__ __launch_bounds__(TPB) void k_from_f64(int64_t n, const double* __restrict__ a, T* __restrict__ b) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) b[i] = (T)a[i];
-}
-template <typename T>
-__global__ __launch_bounds__(TPB) void k_to_f64(int64_t n, const T* __restrict__ a, double* __restrict__ b) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) b[i] = (double)a[i];
-}
-
 Dims dims_of(const fs_ctx* c, int a) { return {{c->fdim[a][0], c->fdim[a][1], c->fdim[a][2]}}; }
 
 // Scratch of one reverse pass (context precision T; sizes in elements).
@@ -596,8 +585,9 @@ int upload_particles(fs_ctx* c, const double* aos, DBuf* dst) {
     for (int d = 0; d < 3; d++) FS_HIP(c, hipMemsetAsync(dst[d].p, 0, (size_t)n * sizeof(T), c->stream));
     return FS_OK;
   }
-  FS_HIP(c, hipMemcpyAsync(c->staging.p, aos, (size_t)n * 3 * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  k_split3<T><<<blocks(n), TPB, 0, c->stream>>>(n, c->staging.as<double>(), dst[0].as<T>(), dst[1].as<T>(),
+  const FsXfer x{c->staging.p, const_cast<double*>(aos), (size_t)n * 3};
+  FS_TRY(fs_xfer_to_device(c, &x, 1, sizeof(T), sizeof(double)));
+  k_split3<T><<<blocks(n), TPB, 0, c->stream>>>(n, c->staging.as<T>(), dst[0].as<T>(), dst[1].as<T>(),
                                                 dst[2].as<T>());
   FS_HIP(c, hipGetLastError());
   FS_HIP(c, hipStreamSynchronize(c->stream));
@@ -609,11 +599,10 @@ int download_particles(fs_ctx* c, DBuf* src, double* aos) {
   const int64_t n = c->np;
   if (!aos) return FS_OK;
   k_join3<T><<<blocks(n), TPB, 0, c->stream>>>(n, src[0].as<T>(), src[1].as<T>(), src[2].as<T>(),
-                                               c->staging.as<double>());
+                                               c->staging.as<T>());
   FS_HIP(c, hipGetLastError());
-  FS_HIP(c, hipMemcpyAsync(aos, c->staging.p, (size_t)n * 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  FS_HIP(c, hipStreamSynchronize(c->stream));
-  return FS_OK;
+  const FsXfer x{c->staging.p, aos, (size_t)n * 3};
+  return fs_xfer_to_host(c, &x, 1, sizeof(T), sizeof(double));
 }
 
 template <typename T>
@@ -667,20 +656,9 @@ int sample_vjp_t(fs_ctx* c, const double* pos, const double* dvel, double* dgrid
   if (st == FS_OK) st = fs_adj_g2p(c, P, c->g, c->g, w.vb, w.xb, w.xb, w.coef);
   c->cfg.advection = adv;
   if (st == FS_OK) st = fs_adj_p2g_sum(c, P, w.coef, w.gb5);
-  for (int a = 0; a < 3 && st == FS_OK; a++) {
-    const int64_t nf = c->n_face[a];
-    DBuf tmp;
-    st = fs_alloc(c, tmp, nf * sizeof(double));
-    if (st != FS_OK) break;
-    k_to_f64<T><<<blocks(nf), TPB, 0, c->stream>>>(nf, w.gb5[a].as<T>(), tmp.as<double>());
-    hipError_t e = hipMemcpyAsync(dgrid[a], tmp.p, nf * sizeof(double), hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    fs_free(tmp);
-    if (e != hipSuccess) {
-      c->set_error(hipGetErrorString(e));
-      st = FS_DEVICE_ERROR;
-    }
-  }
+  FsXfer x[3];
+  for (int a = 0; a < 3; a++) x[a] = {w.gb5[a].p, dgrid[a], (size_t)c->n_face[a]};
+  if (st == FS_OK) st = fs_xfer_to_host(c, x, 3, sizeof(T), sizeof(double));
   w.release();
   return st;
 }
@@ -807,7 +785,9 @@ int fs_sample_grid(fs_ctx* c, const double* pos, const double* u, const double* 
   // PIC G2P of the given grids at the given (or the current) positions; the simulation's
   // particles are left as they were (the face grids are scratch until the next substep)
   const double* src[3] = {u, v, w};
-  for (int a = 0; a < 3; a++) FS_TRY(fs_upload_real(c, c->g[a], src[a], (size_t)c->n_face[a]));
+  FsXfer x[3];
+  for (int a = 0; a < 3; a++) x[a] = {c->g[a].p, const_cast<double*>(src[a]), (size_t)c->n_face[a]};
+  FS_TRY(fs_xfer_to_device(c, x, 3, c->rsz, sizeof(double)));
   DBuf tp[3], tv[3];
   int st = FS_OK;
   for (int d = 0; d < 3 && st == FS_OK; d++) {

@@ -100,6 +100,7 @@ void release_all(fs_ctx* c) {
   fs_pcg_release(c);
   fs_mg_release(c);
   fs_adj_release(c);
+  fs_xfer_release(c);
 }
 
 struct NamedArray {
@@ -164,19 +165,19 @@ float elapsed(hipEvent_t a, hipEvent_t b) {
 
 }  // namespace
 
-// APIC affine rows: device layout [3a + d][particle] at storage width <-> AoS doubles
-// [particle][a][d] across the ABI.
+// APIC affine rows: device layout [3a + d][particle] <-> AoS [particle][a][d] across the ABI, both
+// at storage width (the host copy converts).
 template <typename T>
-__global__ void k_apic_to_aos(int64_t n, const T* __restrict__ cm, double* __restrict__ out) {
+__global__ void k_apic_to_aos(int64_t n, const T* __restrict__ cm, T* __restrict__ out) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= n) return;
-  for (int q = 0; q < 9; q++) out[9 * i + q] = (double)cm[q * n + i];
+  for (int q = 0; q < 9; q++) out[9 * i + q] = cm[q * n + i];
 }
 template <typename T>
-__global__ void k_apic_from_aos(int64_t n, const double* __restrict__ in, T* __restrict__ cm) {
+__global__ void k_apic_from_aos(int64_t n, const T* __restrict__ in, T* __restrict__ cm) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= n) return;
-  for (int q = 0; q < 9; q++) cm[q * n + i] = (T)in[9 * i + q];
+  for (int q = 0; q < 9; q++) cm[q * n + i] = in[9 * i + q];
 }
 
 extern "C" {
@@ -353,14 +354,11 @@ int fs_set_particles(fs_ctx* c, const double* pos, const double* vel, int64_t n)
     return FS_BAD_ARG;
   }
   const double ext[3] = {c->nx * c->h[0], c->ny * c->h[1], c->nz * c->h[2]};
-  for (int64_t i = 0; i < n; i++)
-    for (int d = 0; d < 3; d++) {
-      double p = pos[3 * i + d];
-      if (!(p >= 0.0 && p <= ext[d])) {
-        c->set_error("particle " + std::to_string(i) + " lies outside the domain");
-        return FS_BAD_ARG;
-      }
-    }
+  const int64_t bad = fs_first_outside(pos, 3 * n, ext);
+  if (bad < 3 * n) {
+    c->set_error("particle " + std::to_string(bad / 3) + " lies outside the domain");
+    return FS_BAD_ARG;
+  }
   FS_HIP(c, hipStreamSynchronize(c->stream));
   fs_adj_release(c);  // a recorded rollout refers to the previous particles
   fs_free(c->apicc);  // APIC affine rows restart at zero
@@ -382,7 +380,7 @@ int fs_set_particles(fs_ctx* c, const double* pos, const double* vel, int64_t n)
       FS_TRY(fs_alloc(c, c->pos[d], (size_t)n * c->rsz));
       FS_TRY(fs_alloc(c, c->vel[d], (size_t)n * c->rsz));
     }
-    FS_TRY(fs_alloc(c, c->staging, (size_t)n * 3 * sizeof(double)));
+    FS_TRY(fs_alloc(c, c->staging, (size_t)n * 6 * c->rsz));
     // P2G: one buffer set for the three face grids together, or two sets of one face grid each
     const bool batch = fs_p2g_batch(n);
     const size_t nr = (size_t)n * (batch ? 3 : 1);
@@ -414,20 +412,19 @@ int fs_get_particle_affine(fs_ctx* c, double* c9) {
   if (c->np == 0) return FS_OK;
   FS_TRY(fs_ensure_apic(c));
   DBuf tmp;
-  FS_TRY(fs_alloc(c, tmp, (size_t)c->np * 9 * sizeof(double)));
+  FS_TRY(fs_alloc(c, tmp, (size_t)c->np * 9 * c->rsz));
   const int nb = (int)((c->np + 255) / 256);
-  if (c->mixed) k_apic_to_aos<float><<<nb, 256, 0, c->stream>>>(c->np, c->apicc.as<float>(), tmp.as<double>());
+  if (c->mixed) k_apic_to_aos<float><<<nb, 256, 0, c->stream>>>(c->np, c->apicc.as<float>(), tmp.as<float>());
   else k_apic_to_aos<double><<<nb, 256, 0, c->stream>>>(c->np, c->apicc.as<double>(), tmp.as<double>());
   hipError_t e = hipGetLastError();
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(c9, tmp.p, (size_t)c->np * 9 * sizeof(double), hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  int st = FS_OK;
+  if (e == hipSuccess) st = fs_download_real(c, tmp, c9, (size_t)c->np * 9);
   fs_free(tmp);
   if (e != hipSuccess) {
     c->set_error(hipGetErrorString(e));
     return FS_DEVICE_ERROR;
   }
-  return FS_OK;
+  return st;
 }
 
 int fs_set_particle_affine(fs_ctx* c, const double* c9) {
@@ -436,21 +433,22 @@ int fs_set_particle_affine(fs_ctx* c, const double* c9) {
   if (c->np == 0) return FS_OK;
   FS_TRY(fs_ensure_apic(c));
   DBuf tmp;
-  FS_TRY(fs_alloc(c, tmp, (size_t)c->np * 9 * sizeof(double)));
-  hipError_t e = hipMemcpyAsync(tmp.p, c9, (size_t)c->np * 9 * sizeof(double), hipMemcpyHostToDevice, c->stream);
+  FS_TRY(fs_alloc(c, tmp, (size_t)c->np * 9 * c->rsz));
+  const int st = fs_upload_real(c, tmp, c9, (size_t)c->np * 9);
   const int nb = (int)((c->np + 255) / 256);
-  if (e == hipSuccess) {
-    if (c->mixed) k_apic_from_aos<float><<<nb, 256, 0, c->stream>>>(c->np, tmp.as<double>(), c->apicc.as<float>());
+  hipError_t e = hipSuccess;
+  if (st == FS_OK) {
+    if (c->mixed) k_apic_from_aos<float><<<nb, 256, 0, c->stream>>>(c->np, tmp.as<float>(), c->apicc.as<float>());
     else k_apic_from_aos<double><<<nb, 256, 0, c->stream>>>(c->np, tmp.as<double>(), c->apicc.as<double>());
     e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   }
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   fs_free(tmp);
   if (e != hipSuccess) {
     c->set_error(hipGetErrorString(e));
     return FS_DEVICE_ERROR;
   }
-  return FS_OK;
+  return st;
 }
 
 int fs_set_advector(fs_ctx* c, int32_t method) {
@@ -735,9 +733,8 @@ int fs_get_array(fs_ctx* c, const char* name, void* out) {
   size_t n = (size_t)na.dims[0] * na.dims[1] * na.dims[2];
   if (std::string(name) == "mic_e") return fs_pcg_export_e(c, static_cast<double*>(out));
   if (na.u8) {
-    FS_HIP(c, hipMemcpyAsync(out, na.buf->p, n, hipMemcpyDeviceToHost, c->stream));
-    FS_HIP(c, hipStreamSynchronize(c->stream));
-    return FS_OK;
+    const FsXfer x{na.buf->p, out, n};
+    return fs_xfer_to_host(c, &x, 1, 1, 1);
   }
   return fs_download_real(c, *na.buf, static_cast<double*>(out), n);
 }
@@ -753,13 +750,10 @@ int fs_set_array(fs_ctx* c, const char* name, const void* in) {
   size_t n = (size_t)na.dims[0] * na.dims[1] * na.dims[2];
   c->pcg.built = false;
   if (na.u8) {
-    FS_HIP(c, hipMemcpyAsync(na.buf->p, in, n, hipMemcpyHostToDevice, c->stream));
-    FS_HIP(c, hipStreamSynchronize(c->stream));
-    return FS_OK;
+    const FsXfer x{na.buf->p, const_cast<void*>(in), n};
+    return fs_xfer_to_device(c, &x, 1, 1, 1);
   }
-  int s = fs_upload_real(c, *na.buf, static_cast<const double*>(in), n);
-  if (s == FS_OK) FS_HIP(c, hipStreamSynchronize(c->stream));
-  return s;
+  return fs_upload_real(c, *na.buf, static_cast<const double*>(in), n);
 }
 
 int fs_synchronize(fs_ctx* c) {

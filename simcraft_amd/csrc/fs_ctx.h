@@ -134,6 +134,14 @@ struct AdjTape {
 };
 enum AdjPoint { ADJ_INPUT, ADJ_ADVECTED, ADJ_P2G, ADJ_DIRICHLET, ADJ_BUILT, ADJ_FINAL };
 
+// One lane of a host copy (fs_xfer.hip): two pinned slots and the events of their last copies.
+constexpr int FS_XFER_LANES = 8;
+struct XferLane {
+  void* slot[2] = {nullptr, nullptr};  // two halves of one allocation
+  hipEvent_t ev[2];
+  bool ev_ok[2] = {false, false};
+};
+
 struct fs_ctx {
   fs_config cfg{};
   int device = 0;
@@ -150,7 +158,7 @@ struct fs_ctx {
   // particles (SoA)
   int64_t np = 0;
   DBuf pos[3], vel[3];
-  DBuf staging;  // AoS upload/download
+  DBuf staging;  // AoS upload/download: positions, then velocities, in the storage type
   // face grids: current, ping-pong buffer, valid flags, P2G weight sums, FLIP copy, solid weights
   DBuf g[3], gbuf[3], gvalid[3], gvalidbuf[3], gw[3], glast[3], gweights[3];
   // cell-centred
@@ -205,6 +213,8 @@ struct fs_ctx {
   int64_t n_active_last = 0;
   AdjTape tape;
 
+  XferLane xfer[FS_XFER_LANES];  // pinned slots of host copies, opened on first use
+
   void set_error(const std::string& s) { err = s; }
 };
 
@@ -257,6 +267,19 @@ void fs_mg_release(fs_ctx* c);
 int fs_particles_upload(fs_ctx* c, const double* pos, const double* vel);
 int fs_particles_download(fs_ctx* c, double* pos, double* vel);
 
+// Copies between host arrays and device memory, in order on the context's stream, complete on
+// return: n elements of edev bytes on the device and ehost bytes on the host (equal, or FP32 on the
+// device and FP64 on the host). A copy with a null host pointer is skipped.
+struct FsXfer {
+  void* dev;
+  void* host;
+  size_t n;
+};
+int fs_xfer_to_host(fs_ctx* c, const FsXfer* x, int nx, size_t edev, size_t ehost);
+int fs_xfer_to_device(fs_ctx* c, const FsXfer* x, int nx, size_t edev, size_t ehost);
+void fs_xfer_release(fs_ctx* c);
+// Index of the first of n values outside [0, ext[i % 3]] (or NaN), n if there is none.
+int64_t fs_first_outside(const double* p, int64_t n, const double ext[3]);
 // Conversions between the FP64 ABI and device storage of a given real size.
 int fs_upload_real(fs_ctx* c, DBuf& dst, const double* src, size_t n);
 int fs_download_real(fs_ctx* c, const DBuf& src, double* dst, size_t n);

@@ -1779,33 +1779,22 @@ __global__ __launch_bounds__(TPB) void k_maxabs(int n, const T* __restrict__ g, 
 }
 
 template <typename T>
-__global__ __launch_bounds__(TPB) void k_to_double(int64_t n, const T* __restrict__ a, double* __restrict__ b) {
-  int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) b[i] = (double)a[i];
-}
-template <typename T>
-__global__ __launch_bounds__(TPB) void k_from_double(int64_t n, const double* __restrict__ a, T* __restrict__ b) {
-  int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) b[i] = (T)a[i];
-}
-
-template <typename T>
-__global__ __launch_bounds__(TPB) void k_split_aos(int64_t n, const double* __restrict__ aos, T* __restrict__ x, T* __restrict__ y,
+__global__ __launch_bounds__(TPB) void k_split_aos(int64_t n, const T* __restrict__ aos, T* __restrict__ x, T* __restrict__ y,
                             T* __restrict__ z) {
   int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= n) return;
-  x[i] = (T)aos[3 * i];
-  y[i] = (T)aos[3 * i + 1];
-  z[i] = (T)aos[3 * i + 2];
+  x[i] = aos[3 * i];
+  y[i] = aos[3 * i + 1];
+  z[i] = aos[3 * i + 2];
 }
 template <typename T>
 __global__ __launch_bounds__(TPB) void k_join_aos(int64_t n, const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ z,
-                           double* __restrict__ aos) {
+                           T* __restrict__ aos) {
   int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= n) return;
-  aos[3 * i] = (double)x[i];
-  aos[3 * i + 1] = (double)y[i];
-  aos[3 * i + 2] = (double)z[i];
+  aos[3 * i] = x[i];
+  aos[3 * i + 1] = y[i];
+  aos[3 * i + 2] = z[i];
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -2864,74 +2853,46 @@ int fs_adj_sdf(fs_ctx* c, AdjStep& t, DBuf& phibar, DBuf& psibar, DBuf* xbar) {
   return FS_DISPATCH(c, adj_sdf_t, t, phibar, psibar, xbar);
 }
 
-int fs_upload_real(fs_ctx* c, DBuf& dst, const double* src, size_t n) {
-  if (!c->mixed) {
-    FS_HIP(c, hipMemcpyAsync(dst.p, src, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    return FS_OK;
+template <typename T>
+static int particles_up(fs_ctx* c, const double* pos, const double* vel) {
+  const int64_t n = c->np;
+  T* st = c->staging.as<T>();
+  const FsXfer x[2] = {{st, const_cast<double*>(pos), (size_t)n * 3}, {st + 3 * n, const_cast<double*>(vel), (size_t)n * 3}};
+  FS_TRY(fs_xfer_to_device(c, x, 2, sizeof(T), sizeof(double)));
+  for (int which = 0; which < 2; which++) {
+    DBuf* dst = which == 0 ? c->pos : c->vel;
+    if (!x[which].host)
+      for (int d = 0; d < 3; d++) FS_TRY(fs_zero(c, dst[d]));
+    else
+      k_split_aos<T><<<fs_blocks(n, TPB), TPB, 0, c->stream>>>(n, st + 3 * n * which, dst[0].as<T>(), dst[1].as<T>(),
+                                                               dst[2].as<T>());
   }
-  DBuf tmp;
-  FS_TRY(fs_alloc(c, tmp, n * sizeof(double)));
-  FS_HIP(c, hipMemcpyAsync(tmp.p, src, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  k_from_double<float><<<fs_blocks((int64_t)n, TPB), TPB, 0, c->stream>>>((int64_t)n, tmp.as<double>(), dst.as<float>());
+  FS_HIP(c, hipGetLastError());
   FS_HIP(c, hipStreamSynchronize(c->stream));
-  fs_free(tmp);
   return FS_OK;
 }
 
-int fs_download_real(fs_ctx* c, const DBuf& src, double* dst, size_t n) {
-  if (!c->mixed) {
-    FS_HIP(c, hipMemcpyAsync(dst, src.p, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    FS_HIP(c, hipStreamSynchronize(c->stream));
-    return FS_OK;
+template <typename T>
+static int particles_down(fs_ctx* c, double* pos, double* vel) {
+  const int64_t n = c->np;
+  T* st = c->staging.as<T>();
+  const FsXfer x[2] = {{st, pos, (size_t)n * 3}, {st + 3 * n, vel, (size_t)n * 3}};
+  for (int which = 0; which < 2; which++) {
+    const DBuf* src = which == 0 ? c->pos : c->vel;
+    if (x[which].host)
+      k_join_aos<T><<<fs_blocks(n, TPB), TPB, 0, c->stream>>>(n, src[0].as<T>(), src[1].as<T>(), src[2].as<T>(),
+                                                              st + 3 * n * which);
   }
-  DBuf tmp;
-  FS_TRY(fs_alloc(c, tmp, n * sizeof(double)));
-  k_to_double<float><<<fs_blocks((int64_t)n, TPB), TPB, 0, c->stream>>>((int64_t)n, src.as<float>(), tmp.as<double>());
-  FS_HIP(c, hipMemcpyAsync(dst, tmp.p, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  FS_HIP(c, hipStreamSynchronize(c->stream));
-  fs_free(tmp);
-  return FS_OK;
+  FS_HIP(c, hipGetLastError());
+  return fs_xfer_to_host(c, x, 2, sizeof(T), sizeof(double));
 }
 
 int fs_particles_upload(fs_ctx* c, const double* pos, const double* vel) {
-  int64_t n = c->np;
-  if (n == 0) return FS_OK;
-  for (int which = 0; which < 2; which++) {
-    const double* src = which == 0 ? pos : vel;
-    DBuf* dst = which == 0 ? c->pos : c->vel;
-    if (!src) {
-      for (int d = 0; d < 3; d++) FS_TRY(fs_zero(c, dst[d]));
-      continue;
-    }
-    FS_HIP(c, hipMemcpyAsync(c->staging.p, src, (size_t)n * 3 * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    if (c->mixed)
-      k_split_aos<float><<<fs_blocks(n, TPB), TPB, 0, c->stream>>>(n, c->staging.as<double>(), dst[0].as<float>(),
-                                                                   dst[1].as<float>(), dst[2].as<float>());
-    else
-      k_split_aos<double><<<fs_blocks(n, TPB), TPB, 0, c->stream>>>(n, c->staging.as<double>(), dst[0].as<double>(),
-                                                                    dst[1].as<double>(), dst[2].as<double>());
-    FS_HIP(c, hipGetLastError());
-    FS_HIP(c, hipStreamSynchronize(c->stream));
-  }
-  return FS_OK;
+  if (c->np == 0) return FS_OK;
+  return FS_DISPATCH(c, particles_up, pos, vel);
 }
 
 int fs_particles_download(fs_ctx* c, double* pos, double* vel) {
-  int64_t n = c->np;
-  if (n == 0) return FS_OK;
-  for (int which = 0; which < 2; which++) {
-    double* dst = which == 0 ? pos : vel;
-    DBuf* src = which == 0 ? c->pos : c->vel;
-    if (!dst) continue;
-    if (c->mixed)
-      k_join_aos<float><<<fs_blocks(n, TPB), TPB, 0, c->stream>>>(n, src[0].as<float>(), src[1].as<float>(),
-                                                                  src[2].as<float>(), c->staging.as<double>());
-    else
-      k_join_aos<double><<<fs_blocks(n, TPB), TPB, 0, c->stream>>>(n, src[0].as<double>(), src[1].as<double>(),
-                                                                   src[2].as<double>(), c->staging.as<double>());
-    FS_HIP(c, hipGetLastError());
-    FS_HIP(c, hipMemcpyAsync(dst, c->staging.p, (size_t)n * 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    FS_HIP(c, hipStreamSynchronize(c->stream));
-  }
-  return FS_OK;
+  if (c->np == 0) return FS_OK;
+  return FS_DISPATCH(c, particles_down, pos, vel);
 }

@@ -375,17 +375,10 @@ int fs_rebuild_surface(fs_ctx* c, int64_t* nverts, int64_t* ntris) {
 
 int fs_get_surface(fs_ctx* c, double* vertices, double* normals, uint32_t* indices) {
   if (!c) return FS_BAD_ARG;
-  if (vertices && c->surf_nv)
-    FS_HIP(c, hipMemcpyAsync(vertices, c->surf_v.p, (size_t)c->surf_nv * 3 * sizeof(double), hipMemcpyDeviceToHost,
-                             c->stream));
-  if (normals && c->surf_nv)
-    FS_HIP(c, hipMemcpyAsync(normals, c->surf_n.p, (size_t)c->surf_nv * 3 * sizeof(double), hipMemcpyDeviceToHost,
-                             c->stream));
-  if (indices && c->surf_nt)
-    FS_HIP(c, hipMemcpyAsync(indices, c->surf_i.p, (size_t)c->surf_nt * 3 * sizeof(uint32_t), hipMemcpyDeviceToHost,
-                             c->stream));
-  FS_HIP(c, hipStreamSynchronize(c->stream));
-  return FS_OK;
+  const FsXfer x[2] = {{c->surf_v.p, vertices, (size_t)c->surf_nv * 3}, {c->surf_n.p, normals, (size_t)c->surf_nv * 3}};
+  FS_TRY(fs_xfer_to_host(c, x, 2, sizeof(double), sizeof(double)));
+  const FsXfer t{c->surf_i.p, indices, (size_t)c->surf_nt * 3};
+  return fs_xfer_to_host(c, &t, 1, sizeof(uint32_t), sizeof(uint32_t));
 }
 
 }  // extern "C"
