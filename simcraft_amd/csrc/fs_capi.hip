@@ -93,7 +93,7 @@ void release_all(fs_ctx* c) {
   for (DBuf* b : {&c->surf_v, &c->surf_n, &c->surf_i, &c->apicc}) fs_free(*b);
   for (DBuf* b : {&c->fsdf, &c->fsdfbuf, &c->sdfvalid, &c->sdfvalidbuf, &c->collider, &c->pg, &c->adiag, &c->rhs,
                   &c->active, &c->keys, &c->slots, &c->perm, &c->counts, &c->offs, &c->scan_tmp, &c->red,
-                  &c->recon_tmp, &c->sorted[0], &c->sorted[1], &c->p2g_w,
+                  &c->recon_tmp, &c->sorted[0], &c->sorted[1], &c->p2g_w, &c->p2g_r[0], &c->p2g_r[1],
                   &c->p2g_tiles, &c->offs2, &c->p2g_w2, &c->p2g_tiles2, &c->rkeys, &c->rbinmax, &c->rbins})
     fs_free(*b);
   for (int q = 0; q < 6; q++) fs_free(c->an[q]);
@@ -374,6 +374,7 @@ int fs_set_particles(fs_ctx* c, const double* pos, const double* vel, int64_t n)
     for (int q = 0; q < 2; q++) fs_free(c->sorted[q]);
     fs_free(c->p2g_w);
     fs_free(c->p2g_w2);
+    for (int q = 0; q < 2; q++) fs_free(c->p2g_r[q]);
     fs_free(c->rkeys);
     c->np = 0;
     for (int d = 0; d < 3; d++) {

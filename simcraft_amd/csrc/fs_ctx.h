@@ -168,6 +168,7 @@ struct fs_ctx {
   DBuf keys, slots, perm, counts, offs, scan_tmp;
   DBuf sorted[2];   // bin-ordered velocity component (P2G), one per buffer set
   DBuf p2g_w;       // 12 kernel factors per particle in bin order (P2G)
+  DBuf p2g_r[2];    // APIC: position and affine row per particle in bin order, one per buffer set
   DBuf recon_tmp;   // per-cell squared-distance minima, one array per XCD and a spare (reconstruction)
   DBuf p2g_tiles;   // P2G gather tile work and heaviest-first tile order
   // second P2G buffer set (bin offsets, records, tile order; the velocity records go to

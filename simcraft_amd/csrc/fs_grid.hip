@@ -362,45 +362,6 @@ __global__ __launch_bounds__(TPB) void k_scatter(int n, const int* __restrict__ 
   perm[offs[keys[e]] + slots[e]] = i;
 }
 
-__global__ __launch_bounds__(TPB) void k_sort_bins(int nb, const int* __restrict__ offs, int* __restrict__ perm) {
-  int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nb) return;
-  int s = offs[b], e = offs[b + 1];
-  if (e - s <= 1) return;
-  if (e - s <= 16) {  // in registers: load, sorting network (INT_MAX padding), store
-    int v[16];
-#pragma unroll
-    for (int q = 0; q < 16; q++) v[q] = s + q < e ? perm[s + q] : INT_MAX;
-#pragma unroll
-    for (int size = 2; size <= 16; size <<= 1)
-#pragma unroll
-      for (int stride = size >> 1; stride > 0; stride >>= 1)
-#pragma unroll
-        for (int q = 0; q < 16; q++) {
-          const int r = q ^ stride;
-          if (r > q) {
-            const bool up = (q & size) == 0;
-            const int lo = min(v[q], v[r]), hi = max(v[q], v[r]);
-            v[q] = up ? lo : hi;
-            v[r] = up ? hi : lo;
-          }
-        }
-#pragma unroll
-    for (int q = 0; q < 16; q++)
-      if (s + q < e) perm[s + q] = v[q];
-    return;
-  }
-  for (int i = s + 1; i < e; i++) {
-    int v = perm[i];
-    int j = i - 1;
-    while (j >= s && perm[j] > v) {
-      perm[j + 1] = perm[j];
-      j--;
-    }
-    perm[j + 1] = v;
-  }
-}
-
 // Bin-ordered particle records for the P2G gather: the velocity component and the 12
 // one-dimensional kernel factors N(|p_c - x_node|/h_c) of the 4 nodes per axis around
 // TGrid::nearest, the node weight CubicKernel::weight(h, p - pn) being (wx*wy)*wz. The factors of
@@ -415,13 +376,21 @@ struct P2GVals {
   const T* v[3];
 };
 
-template <typename T>
+// What P2G sums over the particles at a node, with weights w: v w and w (the velocity is their
+// quotient), v w alone (the transposed transfer of the reverse mode), or (v + c.(x_n - x_p)) w and w
+// (APIC, whose records also hold the position and the affine row c: R[0 .. 2] and R[3 .. 5]).
+// APIC at 80^3 mixed, 1 M particles: 0.42 ms for the three face grids and 0.07 ms of records (one
+// thread per node reading its particles from memory took 1.4 ms per face grid).
+enum P2GMode { P2G_NORM, P2G_SUM, P2G_APIC };
+
+template <typename T, bool APIC>
 __global__ __launch_bounds__(TPB) void k_p2g_records(int n, int a0, GridArgs<T> ga,
                                                      const int* __restrict__ perm, const int* __restrict__ keys,
                                                      const int* __restrict__ offs,
                                                      const T* __restrict__ px, const T* __restrict__ py,
                                                      const T* __restrict__ pz, P2GVals<T> vals,
-                                                     P2GVec<T>* __restrict__ W, T* __restrict__ sv) {
+                                                     const T* __restrict__ cm, P2GVec<T>* __restrict__ W,
+                                                     T* __restrict__ sv, T* __restrict__ R) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x, q = blockIdx.y, axis = a0 + q;
   if (i >= n) return;
   const int64_t N = (int64_t)gridDim.y * n;
@@ -439,6 +408,13 @@ __global__ __launch_bounds__(TPB) void k_p2g_records(int n, int a0, GridArgs<T> 
   const T pp[3] = {px[p], py[p], pz[p]};
   const int dims[3] = {ga.nx, ga.ny, ga.nz};
   sv[t] = (axis == 0 ? vals.v[0] : (axis == 1 ? vals.v[1] : vals.v[2]))[p];
+  if constexpr (APIC) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      R[c * N + t] = pp[c];
+      R[(3 + c) * N + t] = cm[(int64_t)(3 * axis + c) * n + p];
+    }
+  }
 #pragma unroll
   for (int c = 0; c < 3; c++) {
     const T off = (c == axis) ? T(0) : T(0.5);
@@ -496,9 +472,10 @@ __device__ __forceinline__ int p2g_slot(int i) { return i + (i >> 3); }
 // stride, so 64 lanes fall into different banks (as 4-vectors the x-factors had 8 lanes to a bank:
 // 56 % of the gather's LDS cycles were conflicts). The y-factors of a slot are one vector where a
 // lane takes four of them (YH >= 4), else arrays as well.
-template <typename T, int YH>
+template <typename T, int YH, bool APIC>
 struct P2GStage {
   static constexpr int CP = P2GCap<T>::padded;
+  T r[APIC ? 6 : 1][APIC ? CP : 1];
   T x[4][CP], z[4][CP], v[CP];
   P2GVec<T> y[YH >= 4 ? CP : 1];
   T ys[YH >= 4 ? 1 : 4][YH >= 4 ? 1 : CP];
@@ -519,9 +496,16 @@ struct P2GStage {
 // when 0 <= j + C <= 3 and takes y-component (y0 + j) mod 4 = (ym + j) mod 4. FP64 forms
 // (wx * wy) * wz, v * w and the sums in the reference's order; FP32 (mixed precision)
 // reassociates to (v wx wz) * wy and (wx wz) * wy, two fused multiply-adds per node.
-template <typename T, bool NORM, int YH, int C>
-__device__ __forceinline__ void p2g_row(const P2GStage<T, YH>& L, int wave, int zm, int ym, int t0, int t1, int c0,
-                                        T (&acc)[YH], T (&ws)[YH]) {
+// APIC forms val = v + ((c0 (-d0) + c1 (-d1)) + c2 (-d2)) with d = x_p - x_n, (wx * wy) * wz and the
+// sums in one order in both precisions; the lane's node lies at nx, ny[j], nz.
+template <typename T, int YH>
+struct P2GNode {
+  T nx, ny[YH], nz;
+};
+template <typename T, P2GMode MODE, int YH, int C>
+__device__ __forceinline__ void p2g_row(const P2GStage<T, YH, MODE == P2G_APIC>& L, const P2GNode<T, YH>& nd, int wave,
+                                        int zm, int ym, int t0, int t1, int c0, T (&acc)[YH], T (&ws)[YH]) {
+  constexpr bool NORM = MODE != P2G_SUM, APIC = MODE == P2G_APIC;
   constexpr int J0 = C < 0 ? -C : 0, J1 = C + YH > 4 ? 4 - C : YH;  // the reached y-nodes [J0, J1)
   constexpr int NW = J1 - J0;
   if (t0 >= t1) return;
@@ -531,6 +515,7 @@ __device__ __forceinline__ void p2g_row(const P2GStage<T, YH>& L, int wave, int 
   struct Op {
     T wx, wz, v;
     P2GVec<T> wy;  // YH >= 4: component (J0 + j) mod 4 of node J0 + j (y0 is a multiple of 4); else [j]
+    T r[APIC ? 6 : 1];
   };
   const T *Lx = L.x[wave], *Lz = L.z[zm];
   auto read = [&](int t) __attribute__((always_inline)) {
@@ -539,6 +524,10 @@ __device__ __forceinline__ void p2g_row(const P2GStage<T, YH>& L, int wave, int 
     o.wx = Lx[s];
     o.wz = Lz[s];
     o.v = L.v[s];
+    if constexpr (APIC) {
+#pragma unroll
+      for (int q = 0; q < 6; q++) o.r[q] = L.r[q][s];
+    }
     if constexpr (YH < 4) {
 #pragma unroll
       for (int j = 0; j < NW; j++) o.wy[j] = L.ys[(ym + J0 + j) & 3][s];
@@ -549,7 +538,17 @@ __device__ __forceinline__ void p2g_row(const P2GStage<T, YH>& L, int wave, int 
   };
   auto sum = [&](const Op& op) __attribute__((always_inline)) {
     const T wx = op.wx, wz = op.wz, v = op.v;
-    if constexpr (sizeof(T) == 4) {
+    if constexpr (APIC) {
+      const T e0 = op.r[3] * (-(op.r[0] - nd.nx)), e2 = op.r[5] * (-(op.r[2] - nd.nz));
+#pragma unroll
+      for (int j = J0; j < J1; j++) {
+        const T w = wx * op.wy[YH < 4 ? j - J0 : j & 3] * wz;
+        const T e1 = op.r[4] * (-(op.r[1] - nd.ny[j]));
+        const T val = v + (e0 + e1 + e2);
+        acc[j] = acc[j] + val * w;
+        ws[j] = ws[j] + w;
+      }
+    } else if constexpr (sizeof(T) == 4) {
       const T xz = wx * wz, vxz = v * xz;
 #pragma unroll
       for (int j = J0; j < J1; j++) {
@@ -568,6 +567,10 @@ __device__ __forceinline__ void p2g_row(const P2GStage<T, YH>& L, int wave, int 
   };
   auto hold = [&](const Op& o) __attribute__((always_inline)) {  // keeps the operands in registers of their own
     asm volatile("" ::"v"(o.wx), "v"(o.wz), "v"(o.v));
+    if constexpr (APIC) {
+#pragma unroll
+      for (int q = 0; q < 6; q++) asm volatile("" ::"v"(o.r[q]));
+    }
     if constexpr (YH < 4) {
 #pragma unroll
       for (int j = 0; j < NW; j++) asm volatile("" ::"v"(o.wy[j]));
@@ -592,11 +595,11 @@ __device__ __forceinline__ void p2g_row(const P2GStage<T, YH>& L, int wave, int 
 }
 
 // p2g_row for the row's y-offset cy (uniform over the wave).
-template <typename T, bool NORM, int YH, int C = 3>
-__device__ __forceinline__ void p2g_rows(const P2GStage<T, YH>& L, int wave, int zm, int ym, int cy, int t0, int t1,
-                                         int c0, T (&acc)[YH], T (&ws)[YH]) {
-  if (cy == C) p2g_row<T, NORM, YH, C>(L, wave, zm, ym, t0, t1, c0, acc, ws);
-  else if constexpr (C > 1 - YH) p2g_rows<T, NORM, YH, C - 1>(L, wave, zm, ym, cy, t0, t1, c0, acc, ws);
+template <typename T, P2GMode MODE, int YH, int C = 3>
+__device__ __forceinline__ void p2g_rows(const P2GStage<T, YH, MODE == P2G_APIC>& L, const P2GNode<T, YH>& nd, int wave,
+                                         int zm, int ym, int cy, int t0, int t1, int c0, T (&acc)[YH], T (&ws)[YH]) {
+  if (cy == C) p2g_row<T, MODE, YH, C>(L, nd, wave, zm, ym, t0, t1, c0, acc, ws);
+  else if constexpr (C > 1 - YH) p2g_rows<T, MODE, YH, C - 1>(L, nd, wave, zm, ym, cy, t0, t1, c0, acc, ws);
 }
 
 // Tile `tile` of a face grid (gx, gy, gz) with bins (bx, by, bz): y-tiles of yh nodes fastest, then
@@ -629,7 +632,7 @@ struct P2GGrids {
     T *G, *Wt, *last;  // sums (or velocities), weight sums, FLIP's copy of the velocities (may be null)
     uint8_t* valid;
   } g[3];
-  int na, ntiles;
+  int a0, na, ntiles;  // face grids a0 .. a0 + na - 1
   __device__ int grid_of(int tile) const { return (na > 1 && tile >= g[1].t0) + (na > 2 && tile >= g[2].t0); }
 };
 
@@ -708,13 +711,15 @@ __global__ __launch_bounds__(1024) void k_p2g_tile_order(int n, const unsigned* 
   }
 }
 
-template <typename T, bool NORM, int YH>
+template <typename T, P2GMode MODE, int YH>
 __global__ __launch_bounds__(P2G_TZ * P2G_WV) void k_p2g_gather(GridArgs<T> ga, P2GGrids<T> gs, int64_t n,
                                                                     const int* __restrict__ order,
                                                                     const P2GVec<T>* __restrict__ W,
-                                                                    const T* __restrict__ vc) {
+                                                                    const T* __restrict__ vc,
+                                                                    const T* __restrict__ R) {
   constexpr int CAP = P2GCap<T>::value;
-  __shared__ P2GStage<T, YH> L;
+  constexpr bool NORM = MODE != P2G_SUM, APIC = MODE == P2G_APIC;
+  __shared__ P2GStage<T, YH, APIC> L;
 
   // Without an order, workgroups go round-robin over the 8 XCDs (id = 8 * k + xcd) and each
   // XCD takes a contiguous run of tiles.
@@ -726,7 +731,8 @@ __global__ __launch_bounds__(P2G_TZ * P2G_WV) void k_p2g_gather(GridArgs<T> ga, 
     const int xcd = blockIdx.x & 7, q = nwg >> 3, r = nwg & 7;
     tile = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (int)(blockIdx.x >> 3);
   }
-  const auto o = gs.g[gs.grid_of(tile)];
+  const int grid = gs.grid_of(tile), axis = gs.a0 + grid;
+  const auto o = gs.g[grid];
   const int gx = o.gx, gy = o.gy, gz = o.gz;
   const int* __restrict__ offs = o.offs;
   T *__restrict__ G = o.G, *__restrict__ Wt = o.Wt, *__restrict__ last = o.last;
@@ -755,13 +761,19 @@ __global__ __launch_bounds__(P2G_TZ * P2G_WV) void k_p2g_gather(GridArgs<T> ga, 
   T acc[YH], ws[YH];
 #pragma unroll
   for (int j = 0; j < YH; j++) acc[j] = ws[j] = T(0);
+  P2GNode<T, YH> nd{};  // APIC: the lane's nodes (nx per slab)
+  if constexpr (APIC) {
+#pragma unroll
+    for (int j = 0; j < YH; j++) nd.ny[j] = coord1(y0 + j, axis == 1 ? T(0) : T(0.5), ga.h[1]);
+    nd.nz = coord1(z, axis == 2 ? T(0) : T(0.5), ga.h[2]);
+  }
   // Rows in walk order: ri = (b0 - xs + 2) * nb1 + (b1 - b1s). While row ri is summed, the
   // first chunk of row ri + 1 is loaded into registers and the bin offsets of row ri + 2 (the
   // row's record range and the lane's range) are read, so no load waits on another.
   const int b1s = g.b1s, nb1 = g.nb1, nrow = g.nrow;
   constexpr int NT = P2G_TZ * P2G_WV, PF = (CAP + NT - 1) / NT;
   P2GVec<T> px[PF], py[PF], pz[PF];
-  T pv[PF];
+  T pv[PF], pr[APIC ? 6 : 1][APIC ? PF : 1];
   struct RowOff {
     int r0, r1, t0, t1;  // the row's records [r0, r1); the lane's, of bins z-2 .. z+1, [t0, t1)
   };
@@ -786,6 +798,10 @@ __global__ __launch_bounds__(P2G_TZ * P2G_WV) void k_p2g_gather(GridArgs<T> ga, 
         py[k] = W[n + pr0 + i];
         pz[k] = W[2 * n + pr0 + i];
         pv[k] = vc[pr0 + i];
+        if constexpr (APIC) {
+#pragma unroll
+          for (int q = 0; q < 6; q++) pr[q][k] = R[q * n + pr0 + i];
+        }
       }
     }
   };
@@ -795,6 +811,7 @@ __global__ __launch_bounds__(P2G_TZ * P2G_WV) void k_p2g_gather(GridArgs<T> ga, 
     const int b0 = xs - 2 + ri / nb1, b1 = b1s + ri % nb1;
     const int xw = b0 - 1 + ((wave - (b0 - 1)) & 3);  // the wave's plane among b0 - 1 .. b0 + 2
     const bool live = xw >= xs && xw < xe;
+    if constexpr (APIC) nd.nx = coord1(xw, axis == 0 ? T(0) : T(0.5), ga.h[0]);
     const int r0 = oc.r0, r1 = oc.r1, lt0 = oc.t0, lt1 = oc.t1, cy = y0 - b1 + 1;
     if (r0 != r1) {
       const int cnt = min(CAP, r1 - r0);
@@ -802,7 +819,13 @@ __global__ __launch_bounds__(P2G_TZ * P2G_WV) void k_p2g_gather(GridArgs<T> ga, 
 #pragma unroll
       for (int k = 0; k < PF; k++) {
         const int i = (int)threadIdx.x + k * NT;
-        if (i < cnt) L.put(p2g_slot(i), px[k], py[k], pz[k], pv[k]);
+        if (i < cnt) {
+          L.put(p2g_slot(i), px[k], py[k], pz[k], pv[k]);
+          if constexpr (APIC) {
+#pragma unroll
+            for (int q = 0; q < 6; q++) L.r[q][p2g_slot(i)] = pr[q][k];
+          }
+        }
       }
       __syncthreads();
     }
@@ -810,14 +833,19 @@ __global__ __launch_bounds__(P2G_TZ * P2G_WV) void k_p2g_gather(GridArgs<T> ga, 
     if (ri + 1 < nrow) fetch(oc);
     on = offsets(ri + 2);
     if (r0 != r1) {
-      if (live) p2g_rows<T, NORM, YH>(L, wave, zm, ym, cy, lt0, min(lt1, r0 + CAP), r0, acc, ws);
+      if (live) p2g_rows<T, MODE, YH>(L, nd, wave, zm, ym, cy, lt0, min(lt1, r0 + CAP), r0, acc, ws);
       for (int c0 = r0 + CAP; c0 < r1; c0 += CAP) {  // a row beyond one chunk: stage the rest in place
         const int cnt = min(CAP, r1 - c0);
         __syncthreads();
-        for (int i = threadIdx.x; i < cnt; i += NT)
+        for (int i = threadIdx.x; i < cnt; i += NT) {
           L.put(p2g_slot(i), W[c0 + i], W[n + c0 + i], W[2 * n + c0 + i], vc[c0 + i]);
+          if constexpr (APIC) {
+#pragma unroll
+            for (int q = 0; q < 6; q++) L.r[q][p2g_slot(i)] = R[q * n + c0 + i];
+          }
+        }
         __syncthreads();
-        if (live) p2g_rows<T, NORM, YH>(L, wave, zm, ym, cy, max(lt0, c0), min(lt1, c0 + CAP), c0, acc, ws);
+        if (live) p2g_rows<T, MODE, YH>(L, nd, wave, zm, ym, cy, max(lt0, c0), min(lt1, c0 + CAP), c0, acc, ws);
       }
     }
     if (ri % nb1 == nb1 - 1 && xw == b0 - 1) {  // plane b0 - 1 has seen every slab b0 - 3 .. b0
@@ -867,9 +895,9 @@ inline P2GShape p2g_tile_shape(int64_t n) {
 }
 
 // Gather of the face grids in gs (arrays set), n records over all of them, on stream st.
-template <typename T, bool NORM>
+template <typename T, P2GMode MODE>
 void launch_p2g_gather(hipStream_t st, GridArgs<T> ga, P2GGrids<T>& gs, int64_t nrec, const P2GVec<T>* W, const T* vc,
-                       DBuf& tiles) {
+                       const T* R, DBuf& tiles) {
   const P2GShape sh = p2g_tile_shape(nrec);
   gs.ntiles = 0;
   for (int q = 0; q < gs.na; q++) {
@@ -888,11 +916,11 @@ void launch_p2g_gather(hipStream_t st, GridArgs<T> ga, P2GGrids<T>& gs, int64_t 
     k_p2g_tile_order<<<1, 1024, 0, st>>>(gs.ntiles, work, ord);
     order = ord;
   }
-  auto go = [&](auto kern) { kern<<<gs.ntiles, P2G_TZ * P2G_WV, 0, st>>>(ga, gs, nrec, order, W, vc); };
-  if (sh.yh == 8) go(k_p2g_gather<T, NORM, 8>);
-  else if (sh.yh == 4) go(k_p2g_gather<T, NORM, 4>);
-  else if (sh.yh == 2) go(k_p2g_gather<T, NORM, 2>);
-  else go(k_p2g_gather<T, NORM, 1>);
+  auto go = [&](auto kern) { kern<<<gs.ntiles, P2G_TZ * P2G_WV, 0, st>>>(ga, gs, nrec, order, W, vc, R); };
+  if (sh.yh == 8) go(k_p2g_gather<T, MODE, 8>);
+  else if (sh.yh == 4) go(k_p2g_gather<T, MODE, 4>);
+  else if (sh.yh == 2) go(k_p2g_gather<T, MODE, 2>);
+  else go(k_p2g_gather<T, MODE, 1>);
 }
 
 // NaiveReconstructor::reconstruct (FluidSim/include/FluidSim/cpu/sdf.h:210-225) as a particle
@@ -1965,55 +1993,8 @@ int ensure_side(fs_ctx* c) {
 // The reference declares AdvectionMethod::APIC without an implementation (setAdvector reaches
 // ERROR, cpu/fluid-simulator.h:96-97). Here each particle carries, per velocity component a, the
 // affine row c_a (the component's gradient near the particle); P2G transfers v_a + c_a.(x_n - x_p)
-// to every node, and G2P sets v_a to the sampled velocity and c_a = D^-1 b over the same nodes, with
-// b = sum w g (x_n - x_p) and D = sum w (x_n - x_p)(x_n - x_p)^T.
-
-// P2G, one thread per node of face grid a: the particles of the bins that reach the node (nearest
-// node b - 1 .. b + 2 around the node, so b in [i-2, i+1] per axis), bins in key order and
-// particles in index order inside a bin - every node sums in (key, index) order, the order of
-// FLIP's P2G. Writes the normalised velocity, the weight sum and the valid flag.
-template <typename T>
-__global__ __launch_bounds__(TPB) void k_p2g_apic(int a, GridArgs<T> ga, int gx, int gy, int gz,
-                                                  const int* __restrict__ offs, const int* __restrict__ perm,
-                                                  const T* __restrict__ px, const T* __restrict__ py,
-                                                  const T* __restrict__ pz, const T* __restrict__ vc,
-                                                  const T* __restrict__ c0, const T* __restrict__ c1,
-                                                  const T* __restrict__ c2, T* __restrict__ G, T* __restrict__ Wt,
-                                                  uint8_t* __restrict__ valid) {
-  const int64_t id = blockIdx.x * (int64_t)TPB + threadIdx.x;
-  if (id >= (int64_t)gx * gy * gz) return;
-  const int k = (int)(id % gz), j = (int)((id / gz) % gy), i = (int)(id / ((int64_t)gz * gy));
-  const T off[3] = {a == 0 ? T(0) : T(0.5), a == 1 ? T(0) : T(0.5), a == 2 ? T(0) : T(0.5)};
-  const T pn[3] = {coord1(i, off[0], ga.h[0]), coord1(j, off[1], ga.h[1]), coord1(k, off[2], ga.h[2])};
-  const int nbk[3] = {ga.nx + 1, ga.ny + 1, ga.nz + 1};  // bin index range of the nearest-node keys
-  const int node[3] = {i, j, k};
-  int lo[3], hi[3];
-#pragma unroll
-  for (int d = 0; d < 3; d++) {
-    lo[d] = max(node[d] - 2, 0);
-    hi[d] = min(node[d] + 1, nbk[d] - 1);
-  }
-  T g = T(0), w_sum = T(0);
-  for (int b0 = lo[0]; b0 <= hi[0]; b0++)
-    for (int b1 = lo[1]; b1 <= hi[1]; b1++)
-      for (int b2 = lo[2]; b2 <= hi[2]; b2++) {
-        const int bin = lin3(b0, b1, b2, nbk[1], nbk[2]);
-        for (int q = offs[bin]; q < offs[bin + 1]; q++) {
-          const int pi = perm[q];
-          const T d0 = px[pi] - pn[0], d1 = py[pi] - pn[1], d2 = pz[pi] - pn[2];  // p - x_n
-          const T w = bspline(wdiv(fabs(d0), ga.h[0])) * bspline(wdiv(fabs(d1), ga.h[1])) *
-                      bspline(wdiv(fabs(d2), ga.h[2]));
-          // x_n - p = -(p - x_n), exactly
-          const T val = vc[pi] + (c0[pi] * (-d0) + c1[pi] * (-d1) + c2[pi] * (-d2));
-          g = g + val * w;
-          w_sum = w_sum + w;
-        }
-      }
-  const bool ok = w_sum > T(0);
-  G[id] = ok ? g / w_sum : T(0);
-  Wt[id] = w_sum;
-  valid[id] = ok ? 1 : 0;
-}
+// to every node (P2G_APIC above), and G2P sets v_a to the sampled velocity and c_a = D^-1 b over the
+// same nodes, with b = sum w g (x_n - x_p) and D = sum w (x_n - x_p)(x_n - x_p)^T.
 
 // G2P: per particle and component, the sampled velocity and the affine row (same nodes, weights
 // and order as sampleVelocity, util.cc:40-85).
@@ -2093,28 +2074,6 @@ __global__ __launch_bounds__(TPB) void k_g2p_apic(int n, GridArgs<T> ga, Grids3<
   }
 }
 
-template <typename T>
-int p2g_apic_t(fs_ctx* c) {
-  GridArgs<T> ga = grid_args<T>(c);
-  const int n = (int)c->np;
-  const int nb = (c->nx + 1) * (c->ny + 1) * (c->nz + 1);
-  FS_TRY(fs_ensure_apic(c));
-  FS_TRY(ensure_bins(c, (size_t)nb + 1));
-  const T* cm = c->apicc.as<T>();
-  for (int a = 0; a < 3; a++) {
-    FS_TRY(bin_particles<T>(c, c->pos, a, 1, c->offs));
-    k_sort_bins<<<fs_blocks(nb, TPB), TPB, 0, c->stream>>>(nb, c->offs.as<int>(), c->perm.as<int>());
-    const int64_t nf = c->n_face[a];
-    k_p2g_apic<T><<<fs_blocks(nf, TPB), TPB, 0, c->stream>>>(
-        a, ga, c->fdim[a][0], c->fdim[a][1], c->fdim[a][2], c->offs.as<int>(), c->perm.as<int>(), c->pos[0].as<T>(),
-        c->pos[1].as<T>(), c->pos[2].as<T>(), c->vel[a].as<T>(), cm + (int64_t)(3 * a) * n,
-        cm + (int64_t)(3 * a + 1) * n, cm + (int64_t)(3 * a + 2) * n, c->g[a].as<T>(), c->gw[a].as<T>(),
-        c->gvalid[a].as<uint8_t>());
-    FS_HIP(c, hipGetLastError());
-  }
-  return FS_OK;
-}
-
 // Sums of val over the face grids from particles at pos, the arrays of face grid a given by set(a):
 // the transfer of P2G (NORM) or its unnormalised sum. With `batch` (fs_p2g_batch, up to 2^22 particles)
 // the three face grids share one binning and one gather. Otherwise each has its own, which needs a
@@ -2122,7 +2081,7 @@ int p2g_apic_t(fs_ctx* c) {
 // face grid a + 1 is binned on the main one (two buffer sets, alternating); the main stream waits
 // for the gathers before the stage ends. Stage at 90^3 mixed: batched 0.37 ms; at 256^3 mixed the
 // overlapped one 4.9 ms (5.9 with a shared binning, which leaves nothing beside the first gather).
-template <typename T, bool NORM, class SET>
+template <typename T, P2GMode MODE, class SET>
 int p2g_run(fs_ctx* c, const DBuf* pos, const DBuf* val, bool overlap, bool batch, SET set) {
   GridArgs<T> ga = grid_args<T>(c);
   const int n = (int)c->np, nb = (c->nx + 1) * (c->ny + 1) * (c->nz + 1);
@@ -2130,6 +2089,8 @@ int p2g_run(fs_ctx* c, const DBuf* pos, const DBuf* val, bool overlap, bool batc
   // the shared bins have to fit 32-bit indices (grids beyond 890^3 take the face grids one by one)
   const int na = batch && 3 * ((int64_t)nb + 1) < ((int64_t)1 << 31) ? 3 : 1;
   overlap = overlap && !batch;
+  constexpr bool APIC = MODE == P2G_APIC;
+  if (APIC) FS_TRY(fs_ensure_apic(c));
   FS_TRY(ensure_bins(c, (size_t)na * (nb + 1)));
   if (overlap) FS_TRY(ensure_side(c));
   const size_t tile_bytes = (size_t)(2 * P2G_MAX_TILES + 16) * sizeof(int);
@@ -2140,15 +2101,21 @@ int p2g_run(fs_ctx* c, const DBuf* pos, const DBuf* val, bool overlap, bool batc
     DBuf& offs = set2 ? c->offs2 : c->offs;
     P2GVec<T>* W = (set2 ? c->p2g_w2 : c->p2g_w).as<P2GVec<T>>();
     T* sv = c->sorted[set2].as<T>();
+    DBuf& rb = c->p2g_r[set2];
+    if (APIC && rb.bytes != (size_t)na * n * 6 * sizeof(T)) {
+      fs_free(rb);
+      FS_TRY(fs_alloc(c, rb, (size_t)na * n * 6 * sizeof(T)));
+    }
+    T* R = rb.as<T>();
     if (overlap && a >= 2) FS_HIP(c, hipStreamWaitEvent(c->stream, c->p2g_ev[a - 2], 0));  // set free again
-    const int pf = NORM ? fs_prof_begin(c, FS_KERNEL_P2G,
+    const int pf = MODE == P2G_NORM ? fs_prof_begin(c, FS_KERNEL_P2G,
                                         (double)n * 4 * sizeof(T) + (double)c->n_face[a] * 2 * sizeof(T))
                         : -1;
     FS_TRY(bin_particles<T>(c, pos, a, na, offs));
     if (n > 0)
-      k_p2g_records<T><<<dim3(fs_blocks(n, TPB), na), TPB, 0, c->stream>>>(
+      k_p2g_records<T, APIC><<<dim3(fs_blocks(n, TPB), na), TPB, 0, c->stream>>>(
           n, a, ga, c->perm.as<int>(), c->keys.as<int>(), offs.as<int>(), pos[0].as<T>(), pos[1].as<T>(),
-          pos[2].as<T>(), vals, W, sv);
+          pos[2].as<T>(), vals, APIC ? c->apicc.as<T>() : nullptr, W, sv, R);
     hipStream_t st = c->stream;
     if (overlap) {
       FS_HIP(c, hipEventRecord(c->p2g_ev[3 + a], c->stream));
@@ -2156,6 +2123,7 @@ int p2g_run(fs_ctx* c, const DBuf* pos, const DBuf* val, bool overlap, bool batc
       st = c->side;
     }
     P2GGrids<T> gs{};
+    gs.a0 = a;
     gs.na = na;
     for (int q = 0; q < na; q++) {
       auto& o = gs.g[q];
@@ -2165,7 +2133,7 @@ int p2g_run(fs_ctx* c, const DBuf* pos, const DBuf* val, bool overlap, bool batc
       o.offs = offs.as<int>() + (size_t)q * (nb + 1);
       set(a + q, o);
     }
-    launch_p2g_gather<T, NORM>(st, ga, gs, (int64_t)na * n, W, sv, set2 ? c->p2g_tiles2 : c->p2g_tiles);
+    launch_p2g_gather<T, MODE>(st, ga, gs, (int64_t)na * n, W, sv, R, set2 ? c->p2g_tiles2 : c->p2g_tiles);
     fs_prof_end(c, pf);
     FS_HIP(c, hipGetLastError());
     if (overlap) FS_HIP(c, hipEventRecord(c->p2g_ev[a], c->side));
@@ -2181,15 +2149,17 @@ int p2g_run(fs_ctx* c, const DBuf* pos, const DBuf* val, bool overlap, bool batc
 // gather of its own on the main stream, so that the timed intervals hold the whole stage.
 template <typename T>
 int p2g_t(fs_ctx* c) {
-  if (c->cfg.advection == FS_ADVECT_APIC) return p2g_apic_t<T>(c);
   const bool timed = c->cfg.profile_stages >= 2 && c->ktime_on;
   const bool flip = c->cfg.advection == FS_ADVECT_FLIP;
-  return p2g_run<T, true>(c, c->pos, c->vel, !timed, !timed && fs_p2g_batch(c->np), [&](int a, auto& o) {
+  auto set = [&](int a, auto& o) {
     o.G = c->g[a].as<T>();
     o.Wt = c->gw[a].as<T>();
     o.valid = c->gvalid[a].as<uint8_t>();
     o.last = flip ? c->glast[a].as<T>() : nullptr;
-  });
+  };
+  const bool batch = !timed && fs_p2g_batch(c->np);
+  if (c->cfg.advection == FS_ADVECT_APIC) return p2g_run<T, P2G_APIC>(c, c->pos, c->vel, !timed, batch, set);
+  return p2g_run<T, P2G_NORM>(c, c->pos, c->vel, !timed, batch, set);
 }
 
 template <typename T>
@@ -2762,7 +2732,7 @@ Grids3<T> grids3(const fs_ctx* c, DBuf* b) {
 // transfer), binned like P2G so the sums are deterministic.
 template <typename T>
 int p2g_sum_t(fs_ctx* c, DBuf* pos, DBuf* coef, DBuf* out) {
-  return p2g_run<T, false>(c, pos, coef, false, fs_p2g_batch(c->np), [&](int a, auto& o) {
+  return p2g_run<T, P2G_SUM>(c, pos, coef, false, fs_p2g_batch(c->np), [&](int a, auto& o) {
     o.G = out[a].as<T>();
     o.Wt = nullptr;
     o.valid = nullptr;

@@ -65,3 +65,40 @@ def test_p2g_tile_shapes(hip, oracle, count, nz, precision):
         mask = w > 1e-2 * max(float(w.max()), 1e-30)  # a node only grazed by a stencil has no accurate quotient
         if mask.any():
             assert float(np.abs(a - b)[mask].max()) <= tol * scale, nm
+
+
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("count,nz", [(0, 33), (3, 33), (20_000, 33), (250_000, 65), (500_000, 33), (2_000_000, 33)])
+def test_p2g_apic_tile_shapes(hip, oracle, count, nz, precision):
+    """APIC's P2G over the same tiles, with the affine rows that G2P takes from random face grids. (Mixed
+    precision: nodes four or more from every wall; a stencil cut by a wall has an ill-conditioned D.)"""
+    n = 21
+    announce(f"apic p2g shapes count={count} nz={nz} precision={precision}")
+    kw = dict(nx=n, ny=n, nz=nz, size_z=nz / n, advection=hip.ADVECT_APIC)
+    pos, vel = scene(count, n, nz)
+    if precision:
+        pos, vel = pos.astype(np.float32).astype(np.float64), vel.astype(np.float32).astype(np.float64)
+        pos = np.minimum(pos, np.array([1.0, 1.0, nz / n]))
+    g = hip.FluidSim(hip.default_config(precision=precision, **kw))
+    o = oracle.OracleSim(oracle.default_config(**kw))
+    for s in (g, o):
+        s.set_particles(pos, vel)
+        for nm in ("u", "v", "w"):
+            shape, _ = g.array_info(nm)
+            s.set(nm, np.random.default_rng(len(nm) + shape[0]).uniform(-1.0, 1.0, shape).astype(np.float32))
+        s.g2p(0.0)
+        s.clear()  # the oracle adds to the grids it finds
+        s.p2g(0.0)
+    inner = (slice(4, -4),) * 3
+    for nm in ("u", "v", "w", "uw", "vw", "ww", "u_valid", "v_valid", "w_valid"):
+        a, b = g.get(nm), o.get(nm)
+        if not precision:
+            assert np.array_equal(a, b), nm
+        elif not nm.endswith("valid"):
+            # terms as above; an affine row comes from 64 nodes and reaches two cells
+            terms = 64 * max(1, int(count / 50 + 16 * count / (n * n * nz)))
+            tol = 4.0 * (terms + 64) * 2.0 ** -24 + 1e-5
+            w = o.get(nm[0] + "w")[inner]
+            mask = w > 1e-2 * max(float(w.max()), 1e-30)
+            if mask.any():
+                assert float(np.abs(a - b)[inner][mask].max()) <= tol * max(float(np.abs(b).max()), 1e-30), nm
