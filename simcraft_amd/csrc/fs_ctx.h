@@ -61,7 +61,7 @@ struct PcgState {
   std::vector<int> live_host;    // brick -> live index or -1
   DBuf live_map;                 // int[nbi*nbj]
   DBuf brick_ij;                 // int2[nlive]
-  DBuf fwd_order, bwd_order;     // int[nlive]: dependency order (anti-diagonal) and its reverse
+  DBuf bricks;                   // Brick[3 nlive]: by live index, in dependency order (anti-diagonal), in its reverse
   DBuf brick_flag;               // int[nbi*nbj]
   // packed system (element layout)
   DBuf adiag, al, ad, ab, nbm, rhs;

@@ -278,8 +278,7 @@ __global__ __launch_bounds__(TH) void k_mg_post2(Lv<S> L, const B* __restrict__ 
   const double bs = block_sum256(acc, sm);
   if (threadIdx.x == 0) xstore(part + blockIdx.x, bs);
   if (blockIdx.x == gridDim.x - 1) {
-    gather_wait256(part, nchunks, sc);
-    const double sig = gather_tree256(part, nchunks, sm);
+    const double sig = gather256(part, nullptr, nchunks, sm, sc).sum;
     if (threadIdx.x == 0) {
       if (!FIRST) sc->beta = sig / sc->sigma;
       sc->sigma = sig;
@@ -429,10 +428,8 @@ __global__ __launch_bounds__(256) void k_mg_init(int64_t n, const uint8_t* __res
     atomicAdd(&sc->n_active, (unsigned long long)bn);
   }
   if (blockIdx.x == gridDim.x - 1) {
-    gather_wait256(part, nchunks, sc);
-    gather_wait256(part2, nchunks, sc);
-    const double tot = gather_tree256(part, nchunks, sm);
-    const double mxx = gather_max256(part2, nchunks, sm);
+    const GatherSumMax red = gather256(part, part2, nchunks, sm, sc);
+    const double tot = red.sum, mxx = red.max;
     if (threadIdx.x == 0) {
       sc->bnorm2sq = tot;
       sc->rnorm2sq = tot;
@@ -475,8 +472,7 @@ __global__ __launch_bounds__(TH) void k_mg_spmv(Lv<S> L, const uint8_t* __restri
   const double bs = block_sum256(acc, sm);
   if (threadIdx.x == 0) xstore(part + blockIdx.x, bs);
   if (blockIdx.x == gridDim.x - 1) {
-    gather_wait256(part, nchunks, sc);
-    const double sdott = gather_tree256(part, nchunks, sm);
+    const double sdott = gather256(part, nullptr, nchunks, sm, sc).sum;
     if (threadIdx.x == 0) {
       sc->sdotz = sdott;
       if (sdott == 0.0) {
@@ -521,10 +517,8 @@ __global__ __launch_bounds__(TH) void k_mg_update(int64_t n, const uint8_t* __re
     xstore(part2 + blockIdx.x, bm);
   }
   if (blockIdx.x == gridDim.x - 1) {
-    gather_wait256(part, nchunks, sc);
-    gather_wait256(part2, nchunks, sc);
-    const double tot = gather_tree256(part, nchunks, sm);
-    const double mxx = gather_max256(part2, nchunks, sm);
+    const GatherSumMax red = gather256(part, part2, nchunks, sm, sc);
+    const double tot = red.sum, mxx = red.max;
     if (threadIdx.x == 0) {
       sc->residual = mxx;
       sc->rnorm2sq = tot;

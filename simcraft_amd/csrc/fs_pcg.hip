@@ -34,11 +34,18 @@ constexpr int NB_SELF = 1, NB_L = 2, NB_D = 4, NB_B = 8, NB_R = 16, NB_U = 32, N
 constexpr int TF_DO = 1, TF_GL = 2, TF_L1 = 4, TF_L2 = 8, TF_GD = 16, TF_D1 = 32, TF_D2 = 64, TF_GB = 128,
               TF_B1 = 256, TF_B2 = 512;
 
+// A live brick and its live neighbours (-1: none): one 32-byte record, so that a kernel has them
+// after one read. An order table lists the records in the order in which tickets are given out.
+struct alignas(16) Brick {
+  int B, L, R, D, U, pad[3];  // itself, -x, +x, -y, +y
+};
+
 struct Lay {
   int nx, ny, nz, nbi, nbj, S, nlive;
   int64_t ne;
   const int* live;   // brick (I*nbj+J) -> live index or -1
   const int2* bij;   // live index -> (I, J)
+  const Brick* brick;  // live index -> record
 };
 
 __device__ inline int64_t eidx(const Lay& L, int B, int s, int lane) { return ((int64_t)B * L.S + s) * 64 + lane; }
@@ -89,16 +96,11 @@ __device__ inline bool decode(const Lay& L, int64_t e, int& B, int& s, int& a, i
 
 constexpr int U = 8;  // slots per chunk; S is a multiple of U
 
-__device__ inline int take_ticket(uint64_t* ctr, uint64_t base, const int* order, int n) {
-  __shared__ int sB;
-  if (threadIdx.x == 0) {
-    uint64_t t = atomicAdd((unsigned long long*)ctr, 1ull) - base;
-    // a ticket outside [0, n) can only follow a failed launch; clamp it so every access
-    // stays in bounds (the exchange polls then time out and the solve reports an error)
-    sB = order[t < (uint64_t)n ? t : (uint64_t)(n - 1)];
-  }
-  __syncthreads();
-  return sB;
+// The record of ticket t - base. A ticket outside [0, n) can only follow a failed launch; it is
+// clamped so that every access stays in bounds (the exchange polls then time out and the solve
+// reports an error).
+__device__ __forceinline__ Brick ticket_brick(uint64_t t, const Brick* __restrict__ order, int n) {
+  return order[t < (uint64_t)n ? t : (uint64_t)(n - 1)];
 }
 
 // Exchange entry of brick B, face f (0: i-face, 1: j-face), slot s, index w (0..7).
@@ -216,14 +218,14 @@ __global__ __launch_bounds__(64) void k_factor_sweep(Lay L, double sigma, const 
                                                      const double* __restrict__ ab, const uint16_t* __restrict__ tfl,
                                                      const double* __restrict__ tnum, double* __restrict__ E,
                                                      double* X, uint64_t* ticket, uint64_t tbase,
-                                                     const int* __restrict__ order, PcgScalars* sc) {
+                                                     const Brick* __restrict__ order, PcgScalars* sc) {
+  __shared__ Brick sb;
   constexpr int UF = 4;
   static_assert(U % UF == 0, "the slot count is a multiple of U");
   const int lane = threadIdx.x, a = lane >> 3, b = lane & 7;
-  const int B = take_ticket(ticket, tbase, order, L.nlive);
-  const int2 ij = L.bij[B];
-  const int BL = ij.x > 0 ? L.live[(ij.x - 1) * L.nbj + ij.y] : -1;
-  const int BD = ij.y > 0 ? L.live[ij.x * L.nbj + ij.y - 1] : -1;
+  if (threadIdx.x == 0) sb = ticket_brick(atomicAdd((unsigned long long*)ticket, 1ull) - tbase, order, L.nlive);
+  __syncthreads();
+  const int B = sb.B, BL = sb.L, BD = sb.D;
   const int S = L.S;
   const bool cL = a == 0 && BL >= 0, cD = b == 0 && BD >= 0;
   const int64_t base = (int64_t)B * S * 64 + lane;
@@ -366,10 +368,8 @@ __global__ __launch_bounds__(256) void k_init(Lay L, const double* __restrict__ 
     xstore(part2 + blockIdx.x, bm);
   }
   if (blockIdx.x == gridDim.x - 1) {
-    gather_wait256(part, nchunks, sc);
-    gather_wait256(part2, nchunks, sc);
-    const double tot = gather_tree256(part, nchunks, sm);
-    const double mxx = gather_max256(part2, nchunks, sm);
+    const GatherSumMax red = gather256(part, part2, nchunks, sm, sc);
+    const double tot = red.sum, mxx = red.max;
     if (threadIdx.x == 0) {
       sc->bnorm2sq = tot;
       sc->rnorm2sq = tot;
@@ -395,11 +395,11 @@ __device__ inline Group group_of(const Lay& L, int base) {
   const int SL = L.S * 64;
   g.B = base / SL;
   g.s0 = (base - g.B * SL) >> 6;
-  const int2 ij = L.bij[g.B];
-  g.BL = ij.x > 0 ? L.live[(ij.x - 1) * L.nbj + ij.y] : -1;
-  g.BR = ij.x + 1 < L.nbi ? L.live[(ij.x + 1) * L.nbj + ij.y] : -1;
-  g.BD = ij.y > 0 ? L.live[ij.x * L.nbj + ij.y - 1] : -1;
-  g.BU = ij.y + 1 < L.nbj ? L.live[ij.x * L.nbj + ij.y + 1] : -1;
+  const Brick br = L.brick[g.B];
+  g.BL = br.L;
+  g.BR = br.R;
+  g.BD = br.D;
+  g.BU = br.U;
   return g;
 }
 // neighbour elements of element e = (B*S + s)*64 + a*8 + b (the neighbour must be active)
@@ -426,18 +426,14 @@ struct FaceOff {
 template <typename S>
 __device__ __forceinline__ FaceOff face_off(const Lay& L, int B) {
   const int SL = L.S * 64, sz = (int)sizeof(S);
-  const int2 ij = L.bij[B];
-  const int BL = ij.x > 0 ? L.live[(ij.x - 1) * L.nbj + ij.y] : -1;
-  const int BR = ij.x + 1 < L.nbi ? L.live[(ij.x + 1) * L.nbj + ij.y] : -1;
-  const int BD = ij.y > 0 ? L.live[ij.x * L.nbj + ij.y - 1] : -1;
-  const int BU = ij.y + 1 < L.nbj ? L.live[ij.x * L.nbj + ij.y + 1] : -1;
+  const Brick br = L.brick[B];
   // byte offsets modulo 2^32: added to the lane's own offset they wrap to the neighbour's
   auto off = [&](int NB, int d) { return NB >= 0 ? (uint32_t)(((int64_t)(NB - B) * SL + d) * sz) : 0u; };
   FaceOff f;
-  f.dL = off(BL, 7 * 64 + 56);
-  f.dR = off(BR, -7 * 64 - 56);
-  f.dD = off(BD, 7 * 64 + 7);
-  f.dU = off(BU, -7 * 64 - 7);
+  f.dL = off(br.L, 7 * 64 + 56);
+  f.dR = off(br.R, -7 * 64 - 56);
+  f.dD = off(br.D, 7 * 64 + 7);
+  f.dU = off(br.U, -7 * 64 - 7);
   return f;
 }
 // element at byte offset `off` of a brick array (an unsigned 32-bit offset from a scalar base,
@@ -458,7 +454,6 @@ __global__ __launch_bounds__(256) void k_spmv(Lay L, const S* __restrict__ x, co
                                               S* __restrict__ y, double* __restrict__ part, int nchunks,
                                               PcgScalars* sc, int iter) {
   __shared__ double sm[4];
-  if (PCG && sc->converged != STOP_RUN) return;
   // A thread's 16 elements (one per group of 256) are independent until the dot product, which
   // adds them in order. Every neighbour is a byte offset from the element's own: a constant
   // inside the brick, a per-brick constant (FaceOff) across a face, zero when the flag is clear
@@ -477,6 +472,7 @@ __global__ __launch_bounds__(256) void k_spmv(Lay L, const S* __restrict__ x, co
   const bool two = SL >= CH;
   const int B0 = min(chunk * CH, ne - 256) / SL;
   const FaceOff f0 = face_off<S>(L, B0), f1 = face_off<S>(L, min(B0 + 1, L.nlive - 1));
+  if (PCG && sc->converged != STOP_RUN) return;  // read with the flags and the face records
   double acc = 0.0;
 #pragma unroll
   for (int m0 = 0; m0 < 16; m0 += MB) {
@@ -546,8 +542,7 @@ __global__ __launch_bounds__(256) void k_spmv(Lay L, const S* __restrict__ x, co
   double bs = block_sum256(acc, sm);
   if (threadIdx.x == 0) xstore(part + chunk, bs);
   if (chunk == (int)gridDim.x - 1) {
-    gather_wait256(part, nchunks, sc);
-    const double sdotz = gather_tree256(part, nchunks, sm);
+    const double sdotz = gather256(part, nullptr, nchunks, sm, sc).sum;
     if (threadIdx.x == 0) {
       sc->sdotz = sdotz;
       if (sdotz == 0.0) {
@@ -609,10 +604,8 @@ __global__ __launch_bounds__(256) void k_resid(Lay L, const double* __restrict__
     xstore(part2 + blockIdx.x, bm);
   }
   if (blockIdx.x == gridDim.x - 1) {
-    gather_wait256(part, nchunks, sc);
-    gather_wait256(part2, nchunks, sc);
-    const double tot = gather_tree256(part, nchunks, sm);
-    const double mxx = gather_max256(part2, nchunks, sm);
+    const GatherSumMax red = gather256(part, part2, nchunks, sm, sc);
+    const double tot = red.sum, mxx = red.max;
     if (threadIdx.x == 0) {
       sc->residual = mxx;
       sc->rnorm2sq = tot;
@@ -704,7 +697,8 @@ struct SwLds {
   double xr[SW_KX][2][64];                // exchange entries of chunks c % SW_KX, from wave 2
   __align__(8) int loaded;  // chunks loaded by wave 3 and (next word) released by wave 1: one
   int freed;                // 8-byte word, so that wave 0 reads both at once
-  int prog, xready, B, stop;       // slots finished by wave 0 / slots whose entries wave 2 has read
+  Brick brick;                     // this workgroup's brick
+  int prog, xready, stop;          // slots finished by wave 0 / slots whose entries wave 2 has read
   int last;                                  // this brick holds the last ticket (it reduces)
 };
 
@@ -990,7 +984,7 @@ __global__ __launch_bounds__(256) void k_fwd(Lay L, T* __restrict__ r, const T* 
                                              const T* __restrict__ cb, const T* __restrict__ E,
                                              T* __restrict__ q, double* X, double* __restrict__ part2,
                                              double* __restrict__ part, uint64_t* ticket, uint64_t tbase,
-                                             const int* __restrict__ order, PcgScalars* sc, int iter, int tol_mode,
+                                             const Brick* __restrict__ order, PcgScalars* sc, int iter, int tol_mode,
                                              double tol) {
   enum { AR = 0, AL = 1, AD = 2, AB = 3, AE = 4, AT = 5 };  // t last: the plain sweep loads five arrays
   constexpr int NARR = UPDATE ? 6 : 5;
@@ -998,9 +992,7 @@ __global__ __launch_bounds__(256) void k_fwd(Lay L, T* __restrict__ r, const T* 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, a = lane >> 3, b = lane & 7;
   if (threadIdx.x == 0) {
     const uint64_t tk = atomicAdd((unsigned long long*)ticket, 1ull) - tbase;
-    // a ticket outside [0, n) can only follow a failed launch; clamp it so every access
-    // stays in bounds (the exchange polls then time out and the solve reports an error)
-    sh.B = order[tk < (uint64_t)L.nlive ? tk : (uint64_t)(L.nlive - 1)];
+    sh.brick = ticket_brick(tk, order, L.nlive);
     sh.last = tk == (uint64_t)(L.nlive - 1);
     sh.stop = UPDATE && sc->converged != STOP_RUN;
     sh.prog = 0;
@@ -1010,12 +1002,10 @@ __global__ __launch_bounds__(256) void k_fwd(Lay L, T* __restrict__ r, const T* 
   }
   __syncthreads();
   if (sh.stop) return;
-  const int B = __builtin_amdgcn_readfirstlane(sh.B);
+  const int B = __builtin_amdgcn_readfirstlane(sh.brick.B);
   const int S = __builtin_amdgcn_readfirstlane(L.S), NC = S / U;
   const size_t brick = (size_t)B * S * 64, face = (size_t)__builtin_amdgcn_readfirstlane(L.nlive) * S * 8;
-  const int2 ij = L.bij[B];
-  const int BL = __builtin_amdgcn_readfirstlane(ij.x > 0 ? L.live[(ij.x - 1) * L.nbj + ij.y] : -1);
-  const int BD = __builtin_amdgcn_readfirstlane(ij.y > 0 ? L.live[ij.x * L.nbj + ij.y - 1] : -1);
+  const int BL = __builtin_amdgcn_readfirstlane(sh.brick.L), BD = __builtin_amdgcn_readfirstlane(sh.brick.D);
   const double* xn[2] = {BL >= 0 ? X + (size_t)BL * S * 8 : nullptr,  // f 0 entries of the -x neighbour
                          BD >= 0 ? X + face + (size_t)BD * S * 8 : nullptr};
   const double* Z = X + 2 * face;  // zero row: no neighbour, or past the last slot
@@ -1076,10 +1066,8 @@ __global__ __launch_bounds__(256) void k_fwd(Lay L, T* __restrict__ r, const T* 
         xstore(part + B, wsum);
       }
       if (__builtin_amdgcn_readfirstlane(sh.last)) {
-        gather_wait_wave(part2, L.nlive, sc);
-        gather_wait_wave(part, L.nlive, sc);
-        const double res = gather_max_wave(part2, L.nlive);
-        const double rr2 = gather_tree256_wave(part, L.nlive);
+        const GatherSumMax red = gather_wave(part, part2, L.nlive, sc);
+        const double res = red.max, rr2 = red.sum;
         if (lane == 0) {
           sc->residual = res;
           sc->rnorm2sq = rr2;
@@ -1183,14 +1171,14 @@ __global__ __launch_bounds__(256) void k_bwd(Lay L, const T* __restrict__ qv, co
                                              const T* __restrict__ du, const T* __restrict__ df,
                                              const T* __restrict__ E, const T* __restrict__ r,
                                              T* __restrict__ z, double* X, double* __restrict__ part,
-                                             uint64_t* ticket, uint64_t tbase, const int* __restrict__ order,
+                                             uint64_t* ticket, uint64_t tbase, const Brick* __restrict__ order,
                                              PcgScalars* sc) {
   enum { AQ = 0, A1 = 1, A2 = 2, A3 = 3, AE = 4, AR = 5 };
   __shared__ SwLds<T> sh;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, a = lane >> 3, b = lane & 7;
   if (threadIdx.x == 0) {
     const uint64_t tk = atomicAdd((unsigned long long*)ticket, 1ull) - tbase;
-    sh.B = order[tk < (uint64_t)L.nlive ? tk : (uint64_t)(L.nlive - 1)];
+    sh.brick = ticket_brick(tk, order, L.nlive);
     sh.last = tk == (uint64_t)(L.nlive - 1);
     sh.stop = !INIT && sc->converged != STOP_RUN;
     sh.prog = 0;
@@ -1200,12 +1188,10 @@ __global__ __launch_bounds__(256) void k_bwd(Lay L, const T* __restrict__ qv, co
   }
   __syncthreads();
   if (sh.stop) return;
-  const int B = __builtin_amdgcn_readfirstlane(sh.B);
+  const int B = __builtin_amdgcn_readfirstlane(sh.brick.B);
   const int S = __builtin_amdgcn_readfirstlane(L.S), NC = S / U;
   const size_t brick = (size_t)B * S * 64, face = (size_t)__builtin_amdgcn_readfirstlane(L.nlive) * S * 8;
-  const int2 ij = L.bij[B];
-  const int BR = __builtin_amdgcn_readfirstlane(ij.x + 1 < L.nbi ? L.live[(ij.x + 1) * L.nbj + ij.y] : -1);
-  const int BU = __builtin_amdgcn_readfirstlane(ij.y + 1 < L.nbj ? L.live[ij.x * L.nbj + ij.y + 1] : -1);
+  const int BR = __builtin_amdgcn_readfirstlane(sh.brick.R), BU = __builtin_amdgcn_readfirstlane(sh.brick.U);
   const double* xn[2] = {BR >= 0 ? X + (size_t)BR * S * 8 : nullptr,  // f 0 entries of the +x neighbour
                          BU >= 0 ? X + face + (size_t)BU * S * 8 : nullptr};
   const double* Z = X + 2 * face;
@@ -1254,8 +1240,7 @@ __global__ __launch_bounds__(256) void k_bwd(Lay L, const T* __restrict__ qv, co
     const double ws = wave_sum(acc);
     if (lane == 0) xstore(part + B, ws);
     if (__builtin_amdgcn_readfirstlane(sh.last)) {
-      gather_wait_wave(part, L.nlive, sc);
-      const double sig = gather_tree256_wave(part, L.nlive);
+      const double sig = gather_wave(part, nullptr, L.nlive, sc).sum;
       if (lane == 0) {
         if (INIT) {
           sc->sigma = sig;
@@ -1413,6 +1398,7 @@ Lay lay_of(const fs_ctx* c) {
   L.ne = P.ne;
   L.live = P.live_map.as<int>();
   L.bij = P.brick_ij.as<int2>();
+  L.brick = P.bricks.as<Brick>();
   return L;
 }
 
@@ -1527,19 +1513,29 @@ int pcg_build(fs_ctx* c) {
     int du = bij[u].x + bij[u].y, dv = bij[v].x + bij[v].y;
     return du < dv;
   });
-  std::vector<int> rord(ord.rbegin(), ord.rend());
+  // records by live index, then in forward and in backward order
+  auto at = [&](int I, int J) {
+    return I >= 0 && J >= 0 && I < P.nbi && J < P.nbj ? P.live_host[I * P.nbj + J] : -1;
+  };
+  std::vector<Brick> rec(3 * (size_t)P.nlive);
+  for (int q = 0; q < P.nlive; q++) {
+    const int I = bij[q].x, J = bij[q].y;
+    rec[q] = {q, at(I - 1, J), at(I + 1, J), at(I, J - 1), at(I, J + 1), {}};
+  }
+  for (int q = 0; q < P.nlive; q++) {
+    rec[P.nlive + q] = rec[ord[q]];
+    rec[2 * P.nlive + q] = rec[ord[P.nlive - 1 - q]];
+  }
   size_t nl = std::max(P.nlive, 1);
   FS_TRY(realloc_if(c, P.brick_ij, nl * sizeof(int2)));
-  FS_TRY(realloc_if(c, P.fwd_order, nl * sizeof(int)));
-  FS_TRY(realloc_if(c, P.bwd_order, nl * sizeof(int)));
+  FS_TRY(realloc_if(c, P.bricks, 3 * nl * sizeof(Brick)));
   const size_t nent = 2 * nl * (size_t)P.S * 8, nx_ = nent + 64;  // entries + zero row (padded)
   FS_TRY(xbuf_get(c, P.xf, nx_ * sizeof(double)));
   FS_TRY(xbuf_get(c, P.xb, nx_ * sizeof(double)));
   if (P.nlive > 0) {
     FS_HIP(c, hipMemcpyAsync(P.live_map.p, P.live_host.data(), nb * sizeof(int), hipMemcpyHostToDevice, c->stream));
     FS_HIP(c, hipMemcpyAsync(P.brick_ij.p, bij.data(), P.nlive * sizeof(int2), hipMemcpyHostToDevice, c->stream));
-    FS_HIP(c, hipMemcpyAsync(P.fwd_order.p, ord.data(), P.nlive * sizeof(int), hipMemcpyHostToDevice, c->stream));
-    FS_HIP(c, hipMemcpyAsync(P.bwd_order.p, rord.data(), P.nlive * sizeof(int), hipMemcpyHostToDevice, c->stream));
+    FS_HIP(c, hipMemcpyAsync(P.bricks.p, rec.data(), rec.size() * sizeof(Brick), hipMemcpyHostToDevice, c->stream));
   }
   // every exchange entry starts as the sentinel
   k_fill_sentinel<<<fs_blocks((int64_t)nent, 256), 256, 0, c->stream>>>((int64_t)nent, P.xf.as<double>());
@@ -1627,8 +1623,8 @@ int pcg_factor(fs_ctx* c) {
   k_factor_sweep<<<P.nlive, 64, 0, c->stream>>>(L, c->cfg.mic_sigma, P.adiag.as<double>(), P.al.as<double>(),
                                                 P.ad.as<double>(), P.ab.as<double>(), P.tflags.as<uint16_t>(),
                                                 P.tnum.as<double>(), P.e.as<double>(), P.xf.as<double>(),
-                                                tk + SW_FACTOR, P.ticket_base[SW_FACTOR], P.fwd_order.as<int>(),
-                                                P.scal.as<PcgScalars>());
+                                                tk + SW_FACTOR, P.ticket_base[SW_FACTOR],
+                                                P.bricks.as<Brick>() + P.nlive, P.scal.as<PcgScalars>());
   fs_prof_end(c, pf);
   P.ticket_base[SW_FACTOR] += P.nlive;
   FS_HIP(c, hipGetLastError());
@@ -1651,8 +1647,8 @@ int launch_fwd(fs_ctx* c, bool update, int iter) {
   auto go = [&](auto kern) {
     kern<<<P.nlive, 256, 0, c->stream>>>(L, y.r, y.t, y.cl, y.cd, y.cb, y.e, y.q, P.xf.as<double>(),
                                         P.partials2.as<double>(), P.partials.as<double>(), tk + SW_FWD,
-                                        P.ticket_base[SW_FWD], P.fwd_order.as<int>(), P.scal.as<PcgScalars>(), iter,
-                                        c->cfg.tol_mode, c->cfg.cg_tolerance);
+                                        P.ticket_base[SW_FWD], P.bricks.as<Brick>() + P.nlive,
+                                        P.scal.as<PcgScalars>(), iter, c->cfg.tol_mode, c->cfg.cg_tolerance);
   };
   const double bytes = (update ? 8.0 : 6.0) * sizeof(S) * c->n_active_last;
   const int pf = fs_prof_begin(c, FS_KERNEL_MIC_FWD, bytes);
@@ -1673,7 +1669,7 @@ int launch_bwd(fs_ctx* c, bool init) {
   auto go = [&](auto kern) {
     kern<<<P.nlive, 256, 0, c->stream>>>(L, y.q, y.dr, y.du, y.df, y.e, y.r, y.z, P.xb.as<double>(),
                                         P.partials.as<double>(), tk + SW_BWD, P.ticket_base[SW_BWD],
-                                        P.bwd_order.as<int>(), P.scal.as<PcgScalars>());
+                                        P.bricks.as<Brick>() + 2 * P.nlive, P.scal.as<PcgScalars>());
   };
   const int pf = fs_prof_begin(c, FS_KERNEL_MIC_BWD, 7.0 * sizeof(S) * c->n_active_last);
   if (init) go(k_bwd<true, S>);
@@ -1935,7 +1931,7 @@ int fs_pcg_export_e(fs_ctx* c, double* out) {
 
 void fs_pcg_release(fs_ctx* c) {
   PcgState& P = c->pcg;
-  for (DBuf* d : {&P.live_map, &P.brick_ij, &P.fwd_order, &P.bwd_order, &P.brick_flag, &P.adiag, &P.al, &P.ad, &P.ab,
+  for (DBuf* d : {&P.live_map, &P.brick_ij, &P.bricks, &P.brick_flag, &P.adiag, &P.al, &P.ad, &P.ab,
                   &P.nbm, &P.rhs, &P.e, &P.cl, &P.cd, &P.cb, &P.dr, &P.du, &P.df, &P.tflags, &P.tnum, &P.x, &P.r,
                   &P.s, &P.t, &P.q, &P.z, &P.partials, &P.partials2, &P.scal, &P.tickets, &P.f_adiag,
                   &P.f_al, &P.f_ad, &P.f_ab, &P.f_e, &P.f_cl, &P.f_cd, &P.f_cb, &P.f_dr, &P.f_du, &P.f_df, &P.f_r,

@@ -153,81 +153,82 @@ __device__ __forceinline__ double chunk_max(double mx, double* terms) {
   return mx;
 }
 
-// Block-wide wait until p[0, n) are all set; false if the wait gave up.
-__device__ inline bool gather_wait256(const double* p, int n, PcgScalars* sc) {
-  long spins = 0;
-  while (true) {
-    int mine = 1;
-    for (int m = threadIdx.x; m < n; m += blockDim.x) mine &= xunset(xload(p + m)) ? 0 : 1;
-    if (__syncthreads_and(mine)) return true;
-    __builtin_amdgcn_s_sleep(2);
-    int give = 0;
-    if ((++spins & 63) == 0 && threadIdx.x == 0) {
-      const int to = __hip_atomic_load(&sc->wait_timeouts, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      give = (to != 0 || spins > SPIN_LIMIT) ? 1 : 0;
-      if (give) atomicAdd(&sc->wait_timeouts, 1);
-    }
-    if (__syncthreads_or(give)) return false;
-  }
-}
-// Fixed tree over the n gathered entries (thread t sums p[t + 256m] for m ascending, then
-// block_sum256), which it returns to the sentinel.
-__device__ inline double gather_tree256(double* p, int n, double* sm) {
-  double a = 0.0;
-  for (int m = threadIdx.x < 256 ? threadIdx.x : n; m < n; m += 256) {
-    a += xload(p + m);
-    xstore(p + m, xsent());
-  }
-  return block_sum256(a, sm);
-}
-// max over gathered entries (order-free: the comparison never takes a NaN), returned to the sentinel
-__device__ inline double gather_max256(double* p, int n, double* sm) {
-  double mx = 0.0;
-  for (int m = threadIdx.x < 256 ? threadIdx.x : n; m < n; m += 256) {
-    const double v = xload(p + m);
-    mx = (mx < v) ? v : mx;
-    xstore(p + m, xsent());
-  }
-  return block_max256(mx, sm);
-}
-// One wave's wait until p[0, n) are all set; false if the wait gave up.
-__device__ inline bool gather_wait_wave(const double* p, int n, PcgScalars* sc) {
-  const int lane = threadIdx.x & 63;
-  long spins = 0;
-  while (true) {
-    bool mine = true;
-    for (int m = lane; m < n; m += 64) mine &= !xunset(xload(p + m));
-    if (__builtin_amdgcn_ballot_w64(!mine) == 0) return true;
-    __builtin_amdgcn_s_sleep(2);
-    if ((++spins & 63) == 0) {
-      const int to = __hip_atomic_load(&sc->wait_timeouts, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (to != 0 || spins > SPIN_LIMIT) {
-        if (lane == 0) atomicAdd(&sc->wait_timeouts, 1);
-        return false;
+// The last block reads each entry as it waits for it, and keeps the value: a pass that only waits
+// and another that reads again is one more round trip to memory at the end of every kernel that
+// reduces, and nothing else runs by then (us, two passes / one: FP64 SpMV 13.6 / 12.0 at 32^3, forward
+// sweep 17.1 / 16.3; mixed multigrid's update with two arrays 8.0 / 7.4 at 64^3, 41.1 / 34.8 at 256^3,
+// 4096 entries). An entry is returned to the sentinel by the thread that read it. A wait that gives
+// up yields 0 and counts a timeout (the solve then reports FS_DEVICE_ERROR).
+
+// Fixed tree over the n entries of p (thread t < 256 sums p[t + 256 m] for m ascending, then
+// block_sum256) and, where p2 is given, the maximum over p2 (order-free: the comparison never takes
+// a NaN). All threads of the block call.
+struct GatherSumMax {
+  double sum, max;
+};
+__device__ inline GatherSumMax gather256(double* p, double* p2, int n, double* sm, PcgScalars* sc) {
+  constexpr int K = 4;  // entries in flight per thread and array
+  double a = 0.0, mx = 0.0;
+  if (threadIdx.x < 256) {
+    for (int m0 = threadIdx.x; m0 < n; m0 += 256 * K) {
+      double v[K], w[K];
+#pragma unroll
+      for (int q = 0; q < K; q++) {
+        const int m = m0 + 256 * q;
+        v[q] = m < n ? xload(p + m) : 0.0;
+        w[q] = p2 && m < n ? xload(p2 + m) : 0.0;
+      }
+#pragma unroll
+      for (int q = 0; q < K; q++) {
+        const int m = m0 + 256 * q;
+        if (m >= n) continue;
+        a += xpoll(p + m, v[q], sc);
+        xstore(p + m, xsent());
+        if (p2) {
+          const double x = xpoll(p2 + m, w[q], sc);
+          mx = (mx < x) ? x : mx;
+          xstore(p2 + m, xsent());
+        }
       }
     }
   }
+  GatherSumMax r;
+  r.sum = block_sum256(a, sm);
+  r.max = p2 ? block_max256(mx, sm) : 0.0;
+  return r;
 }
-// The same tree evaluated by one 64-lane wave (lane l plays threads l, l+64, l+128, l+192).
-__device__ inline double gather_tree256_wave(double* p, int n) {
-  double w[4];
+// The same by one 64-lane wave (lane l plays threads l, l + 64, l + 128, l + 192).
+__device__ inline GatherSumMax gather_wave(double* p, double* p2, int n, PcgScalars* sc) {
+  const int lane = threadIdx.x & 63;
+  double w[4] = {0.0, 0.0, 0.0, 0.0}, mx = 0.0;
+  for (int m0 = 0; m0 < n; m0 += 256) {
+    double v[4], x[4];
 #pragma unroll
-  for (int v = 0; v < 4; v++) {
-    double a = 0.0;
-    for (int m = (threadIdx.x & 63) + 64 * v; m < n; m += 256) a += xload(p + m);
-    w[v] = wave_sum(a);
+    for (int q = 0; q < 4; q++) {
+      const int m = m0 + 64 * q + lane;
+      v[q] = m < n ? xload(p + m) : 0.0;
+      x[q] = p2 && m < n ? xload(p2 + m) : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int m = m0 + 64 * q + lane;
+      if (m >= n) continue;
+      w[q] += xpoll(p + m, v[q], sc);
+      xstore(p + m, xsent());
+      if (p2) {
+        const double y = xpoll(p2 + m, x[q], sc);
+        mx = (mx < y) ? y : mx;
+        xstore(p2 + m, xsent());
+      }
+    }
   }
-  for (int m = threadIdx.x & 63; m < n; m += 64) xstore(p + m, xsent());
-  return (w[0] + w[1]) + (w[2] + w[3]);
-}
-__device__ inline double gather_max_wave(double* p, int n) {
-  double mx = 0.0;
-  for (int m = threadIdx.x & 63; m < n; m += 64) {
-    const double v = xload(p + m);
-    mx = (mx < v) ? v : mx;
-    xstore(p + m, xsent());
-  }
-  return wave_max(mx);
+  GatherSumMax r;
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    if (64 * q < n) w[q] = wave_sum(w[q]);  // uniform; a sum over no entry is +0
+  r.sum = (w[0] + w[1]) + (w[2] + w[3]);
+  r.max = p2 ? wave_max(mx) : 0.0;
+  return r;
 }
 
 __global__ void k_fill_sentinel(int64_t n, double* __restrict__ x) {
