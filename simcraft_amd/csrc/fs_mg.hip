@@ -45,9 +45,13 @@ constexpr double MG_ALPHA = 1.8;  // coarse-correction weight
 constexpr int MCH = 4096;         // cells per block of the kernels that reduce
 // Up to this many blocks of them take 1024 threads instead of 256 (chunk_sum): with few blocks a
 // thread's sixteen cells in turn are the kernel's time, with many the other blocks hide them. Mixed,
-// us, 256 / 1024 threads, SpMV, last sweep, update: 128^3 38.5 / 15.9, 21.8 / 9.8, 13.4 / 9.0; 192^3
-// (1728 blocks) 52.7 / 34.5, 28.5 / 20.2, 22.2 / 22.4; 256^3 (4096) 75 / 78, 38.4 / 44.2, 41.3 / 50.7.
-constexpr unsigned MG_WIDE = 2048;
+// us, 256 / 1024 threads, SpMV, last sweep, update: 64^3 12.5 / 8.9, 9.3 / 5.6, 8.5 / 7.5; 128^3 (512
+// blocks) 15.0 / 9.8, 10.5 / 6.9, 10.9 / 8.0; 192^3 (1728) 23.6 / 25.1, 14.7 / 16.8, 17.9 / 19.2.
+constexpr unsigned MG_WIDE = 1024;
+// Cells in flight per thread of the 1024-thread forms: with four, FP64 operands spill (SpMV 19.2 us at
+// 128^3, 13.3 with a branch per term).
+template <typename S>
+constexpr int MG_FLIGHT = sizeof(S) == 4 ? 4 : 2;
 
 template <typename S>
 struct Lv {
@@ -65,17 +69,26 @@ __device__ __forceinline__ void decode3(int64_t c, int ny, int nz, int& i, int& 
 
 // Row c of the level's operator applied to xo: diagonal, -x, -y, -z, +x, +y, +z (the order of
 // applyCompressedMatrix, project-solver.cc:23-35); terms outside the grid are dropped. xo(q, i, j, k)
-// gives the operand at cell q = (i, j, k).
+// gives the operand at cell q = (i, j, k). A term outside the grid reads the cell itself and is dropped
+// by a select, so that a thread's reads are in flight together: a branch per term made each wait for
+// the one before it (mixed, us, branches / selects: SpMV 15.6 / 8.9 at 64^3, 73 / 50 at 256^3; last sweep
+// 9.6 / 5.6, 35.6 / 26.0; first sweep 43.5 / 38.2 at 256^3).
 template <typename R, typename S, typename XO>
 __device__ __forceinline__ R row(const Lv<S>& L, int64_t c, int i, int j, int k, XO xo) {
   const int64_t sx = (int64_t)L.ny * L.nz, sy = L.nz;
-  R t = (R)L.D[c] * xo(c, i, j, k);
-  if (i > 0) t = t + (R)L.Cx[c] * xo(c - sx, i - 1, j, k);
-  if (j > 0) t = t + (R)L.Cy[c] * xo(c - sy, i, j - 1, k);
-  if (k > 0) t = t + (R)L.Cz[c] * xo(c - 1, i, j, k - 1);
-  if (i < L.nx - 1) t = t + (R)L.Cx[c + sx] * xo(c + sx, i + 1, j, k);
-  if (j < L.ny - 1) t = t + (R)L.Cy[c + sy] * xo(c + sy, i, j + 1, k);
-  if (k < L.nz - 1) t = t + (R)L.Cz[c + 1] * xo(c + 1, i, j, k + 1);
+  const bool l = i > 0, d = j > 0, b = k > 0, r = i < L.nx - 1, u = j < L.ny - 1, f = k < L.nz - 1;
+  const int64_t cr = r ? c + sx : c, cu = u ? c + sy : c, cf = f ? c + 1 : c;
+  const R kl = (R)L.Cx[c], kd = (R)L.Cy[c], kb = (R)L.Cz[c], kr = (R)L.Cx[cr], ku = (R)L.Cy[cu], kf = (R)L.Cz[cf];
+  const R x0 = xo(c, i, j, k), xl = xo(l ? c - sx : c, i - l, j, k), xd = xo(d ? c - sy : c, i, j - d, k),
+          xb = xo(b ? c - 1 : c, i, j, k - b), xr = xo(cr, i + r, j, k), xu = xo(cu, i, j + u, k),
+          xf = xo(cf, i, j, k + f);
+  R t = (R)L.D[c] * x0;
+  t = l ? t + kl * xl : t;
+  t = d ? t + kd * xd : t;
+  t = b ? t + kb * xb : t;
+  t = r ? t + kr * xr : t;
+  t = u ? t + ku * xu : t;
+  t = f ? t + kf * xf : t;
   return t;
 }
 
@@ -179,7 +192,8 @@ __device__ __forceinline__ S post1_cell(const Lv<S>& L, const B* __restrict__ b,
                                         const S* __restrict__ xc, int cny, int cnz, S alpha, int64_t c, int i, int j,
                                         int k) {
   auto xo = [&](int64_t q, int qi, int qj, int qk) {
-    return L.W[q] > S(0) ? x[q] + alpha * xc[((int64_t)(qi >> 1) * cny + (qj >> 1)) * cnz + (qk >> 1)] : x[q];
+    const S w = L.W[q], v = x[q], p = xc[((int64_t)(qi >> 1) * cny + (qj >> 1)) * cnz + (qk >> 1)];
+    return w > S(0) ? v + alpha * p : v;
   };
   return xo(c, i, j, k) + L.W[c] * ((S)b[c] - row<S>(L, c, i, j, k, xo));
 }
@@ -266,15 +280,28 @@ __global__ __launch_bounds__(TH) void k_mg_post2(Lv<S> L, const B* __restrict__ 
   if (sc && sc->converged != STOP_RUN) return;
   __shared__ double terms[CHUNK_TERMS<TH>];
   const int64_t n = (int64_t)L.nx * L.ny * L.nz;
-  const double acc = chunk_sum<TH>(terms, [&](int e) __attribute__((always_inline)) {
-    const int64_t c = (int64_t)blockIdx.x * MCH + e;
-    if (c >= n || !(L.W[c] > S(0))) return 0.0;  // z = 0 there, and so is its product with r
-    int i, j, k;
-    decode3(c, L.ny, L.nz, i, j, k);
-    const S out = sweep_cell<S, B>(L, b, xs, c, i, j, k);
-    x[c] = out;
-    return (double)out * (double)b[c];
-  });
+  struct V {
+    S out;
+    double b;
+  };
+  const int64_t c0 = (int64_t)blockIdx.x * MCH;
+  auto at = [&](int e) { return c0 + e < n ? c0 + e : n - 1; };
+  const double acc = chunk_sum<TH, V, MG_FLIGHT<S>>(
+      terms,
+      [&](int e) __attribute__((always_inline)) {
+        const S w = L.W[at(e)];  // where it is 0, so are z and its product with r
+        return c0 + e < n && w > S(0);
+      },
+      [&](int e) __attribute__((always_inline)) {
+        const int64_t c = at(e);
+        int i, j, k;
+        decode3(c, L.ny, L.nz, i, j, k);
+        return V{sweep_cell<S, B>(L, b, xs, c, i, j, k), (double)b[c]};
+      },
+      [&](int e, const V& v) __attribute__((always_inline)) {
+        x[c0 + e] = v.out;
+        return (double)v.out * v.b;
+      });
   const double bs = block_sum256(acc, sm);
   if (threadIdx.x == 0) xstore(part + blockIdx.x, bs);
   if (blockIdx.x == gridDim.x - 1) {
@@ -456,19 +483,33 @@ __global__ __launch_bounds__(TH) void k_mg_spmv(Lv<S> L, const uint8_t* __restri
   const int64_t n = (int64_t)L.nx * L.ny * L.nz;
   const bool first = iter == 1;
   const double beta = sc->beta;
-  auto so = [&](int64_t q, int, int, int) { return first ? (double)z[q] : (double)z[q] + beta * s_old[q]; };
+  auto so = [&](int64_t q, int, int, int) {
+    const double zq = (double)z[q], v = zq + beta * s_old[q];
+    return first ? zq : v;
+  };
   __shared__ double terms[CHUNK_TERMS<TH>];
-  const double acc = chunk_sum<TH>(terms, [&](int e) __attribute__((always_inline)) {
-    const int64_t c = (int64_t)blockIdx.x * MCH + e;
-    if (c >= n || !act[c]) return 0.0;
-    int i, j, k;
-    decode3(c, L.ny, L.nz, i, j, k);
-    const double sv = so(c, i, j, k);
-    const double tv = row<double>(L, c, i, j, k, so);
-    s_new[c] = sv;
-    t[c] = tv;
-    return sv * tv;
-  });
+  struct V {
+    double s, t;
+  };
+  const int64_t c0 = (int64_t)blockIdx.x * MCH;
+  auto at = [&](int e) { return c0 + e < n ? c0 + e : n - 1; };
+  const double acc = chunk_sum<TH, V, MG_FLIGHT<S>>(
+      terms,
+      [&](int e) __attribute__((always_inline)) {
+        const uint8_t on = act[at(e)];
+        return c0 + e < n && on != 0;
+      },
+      [&](int e) __attribute__((always_inline)) {
+        const int64_t c = at(e);
+        int i, j, k;
+        decode3(c, L.ny, L.nz, i, j, k);
+        return V{so(c, i, j, k), row<double>(L, c, i, j, k, so)};
+      },
+      [&](int e, const V& v) __attribute__((always_inline)) {
+        s_new[c0 + e] = v.s;
+        t[c0 + e] = v.t;
+        return v.s * v.t;
+      });
   const double bs = block_sum256(acc, sm);
   if (threadIdx.x == 0) xstore(part + blockIdx.x, bs);
   if (blockIdx.x == gridDim.x - 1) {
@@ -499,16 +540,28 @@ __global__ __launch_bounds__(TH) void k_mg_update(int64_t n, const uint8_t* __re
   const double alpha = sc->alpha;
   __shared__ double terms[CHUNK_TERMS<TH>];
   double mx = 0.0;
-  const double ss = chunk_sum<TH>(terms, [&](int e) __attribute__((always_inline)) {
-    const int64_t c = (int64_t)blockIdx.x * MCH + e;
-    if (c >= n || !act[c]) return 0.0;  // r = 0 there
-    x[c] = x[c] + alpha * s[c];
-    const double rv = r[c] + (-alpha) * t[c];
-    r[c] = rv;
-    const double av = fabs(rv);
-    mx = (mx < av) ? av : mx;
-    return rv * rv;
-  });
+  struct V {
+    double x, r;
+  };
+  const int64_t c0 = (int64_t)blockIdx.x * MCH;
+  auto at = [&](int e) { return c0 + e < n ? c0 + e : n - 1; };
+  const double ss = chunk_sum<TH, V, 4>(
+      terms,
+      [&](int e) __attribute__((always_inline)) {
+        const uint8_t on = act[at(e)];  // r = 0 on the others
+        return c0 + e < n && on != 0;
+      },
+      [&](int e) __attribute__((always_inline)) {
+        const int64_t c = at(e);
+        return V{x[c] + alpha * s[c], r[c] + (-alpha) * t[c]};
+      },
+      [&](int e, const V& v) __attribute__((always_inline)) {
+        x[c0 + e] = v.x;
+        r[c0 + e] = v.r;
+        const double av = fabs(v.r);
+        mx = (mx < av) ? av : mx;
+        return v.r * v.r;
+      });
   mx = chunk_max<TH>(mx, terms);
   const double bm = block_max256(mx, sm);
   const double bs = block_sum256(ss, sm);

@@ -111,24 +111,44 @@ __device__ __forceinline__ bool xunset(double v) { return (uint32_t)__double2hii
 // brick with the last ticket) waits until every entry is set, reduces them in the fixed order and
 // stores the sentinel back, so the entries are unset again for the next kernel.
 
-// Sum of the terms f(e), e = 0 .. 4095, of a chunk in the fixed order of 256 threads with 16 elements
-// each (thread t: e = t + 256 m, m ascending), by TH threads; the value is that of the first 256
-// threads. With TH = 1024, thread (g, t) = (tid / 256, tid % 256) evaluates m = 4g .. 4g + 3 and the
-// terms meet in LDS (TERMS<1024> doubles), so that a thread waits for four elements' loads in turn
-// instead of sixteen: the choice where a kernel has too few chunks to hide them by other blocks.
+// Sum of the terms done(e, load(e)) of a chunk's elements e = 0 .. 4095 with live(e) (0 for the others)
+// in the fixed order of 256 threads with 16 elements each (thread t: e = t + 256 m, m ascending), by TH
+// threads; the value is that of the first 256 threads. With TH = 1024, thread (g, t) = (tid / 256,
+// tid % 256) evaluates m = 4g .. 4g + 3 and the terms meet in LDS (TERMS<1024> doubles): the choice
+// where a kernel has too few chunks to hide a thread's sixteen elements in turn by other blocks. There
+// G of the four at a time are loaded before any is stored, unless none of the wave's is live: so load
+// only reads, any element, and done writes.
 template <int TH>
 constexpr int CHUNK_TERMS = TH == 256 ? 1 : 4096;
-template <int TH, class F>
-__device__ __forceinline__ double chunk_sum(double* terms, F&& f) {
+template <int TH, class V, int G, class A, class L, class D>
+__device__ __forceinline__ double chunk_sum(double* terms, A&& live, L&& load, D&& done) {
   double a = 0.0;
   if constexpr (TH == 256) {
 #pragma unroll 1
-    for (int m = 0; m < 16; m++) a += f(256 * m + (int)threadIdx.x);
+    for (int m = 0; m < 16; m++) {
+      const int e = 256 * m + (int)threadIdx.x;
+      a += live(e) ? done(e, load(e)) : 0.0;
+    }
   } else {
     static_assert(TH == 1024, "four groups of 256 threads");
     const int e0 = 1024 * (int)(threadIdx.x >> 8) + (int)(threadIdx.x & 255);
+    bool on[4];
 #pragma unroll
-    for (int q = 0; q < 4; q++) terms[e0 + 256 * q] = f(e0 + 256 * q);
+    for (int q = 0; q < 4; q++) on[q] = live(e0 + 256 * q);
+    double term[4] = {0.0, 0.0, 0.0, 0.0};
+    if (__builtin_amdgcn_ballot_w64(on[0] || on[1] || on[2] || on[3])) {
+#pragma unroll
+      for (int q0 = 0; q0 < 4; q0 += G) {
+        V v[G];
+#pragma unroll
+        for (int q = 0; q < G; q++) v[q] = load(e0 + 256 * (q0 + q));
+#pragma unroll
+        for (int q = 0; q < G; q++)
+          if (on[q0 + q]) term[q0 + q] = done(e0 + 256 * (q0 + q), v[q]);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) terms[e0 + 256 * q] = term[q];
     __syncthreads();
     if (threadIdx.x < 256) {
 #pragma unroll
