@@ -54,7 +54,6 @@ __device__ inline void unlin(int64_t id, const int d[3], int& i, int& j, int& k)
 struct Dims {
   int d[3];
 };
-
 // applyCollider (fluid-simulator.cc:76-111) is u *= 0 on the walls and u *= (1 - n_a) inside
 // the collider: the reverse multiplies by the same factor.
 template <typename T>
@@ -287,7 +286,20 @@ __global__ __launch_bounds__(TPB) void k_force_adj(int a, Dims D, const uint8_t*
 }
 
 // extrapolate (cpu/fluid-simulator.h:204-253): the valid mask after one iteration.
-__global__ __launch_bounds__(TPB) void k_extrap_mask(Dims D, const uint8_t* __restrict__ V, uint8_t* __restrict__ VN) {
+// The face grid is blockIdx.y, as in k_extrap_adj.
+struct MaskPass {
+  Dims D;
+  const uint8_t* V;
+  uint8_t* VN;
+};
+struct MaskPass3 {
+  MaskPass f[3];
+};
+__global__ __launch_bounds__(TPB) void k_extrap_mask(MaskPass3 M) {
+  const MaskPass f = M.f[blockIdx.y];
+  const Dims D = f.D;
+  const uint8_t* __restrict__ V = f.V;
+  uint8_t* __restrict__ VN = f.VN;
   const int64_t id = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (id >= (int64_t)D.d[0] * D.d[1] * D.d[2]) return;
   int i, j, k;
@@ -314,8 +326,25 @@ __device__ inline int valid_count(const uint8_t* V, int64_t id, int i, int j, in
 //   Gbar(n)  = B(n) + [n valid] sum over invalid neighbours c of A(c) / count(c)
 //   GBbar(c) = [c valid] A(c)
 template <typename T>
-__global__ __launch_bounds__(TPB) void k_extrap_adj(Dims D, const uint8_t* __restrict__ V, const T* __restrict__ A, const T* __restrict__ B,
-                             T* __restrict__ Gb, T* __restrict__ GBb) {
+struct ExtrapAdj {
+  Dims D;
+  const uint8_t* V;
+  const T *A, *B;
+  T *Gb, *GBb;
+};
+template <typename T>
+struct ExtrapAdj3 {
+  ExtrapAdj<T> f[3];
+};
+template <typename T>
+__global__ __launch_bounds__(TPB) void k_extrap_adj(ExtrapAdj3<T> X) {
+  const ExtrapAdj<T> f = X.f[blockIdx.y];
+  const Dims D = f.D;
+  const uint8_t* __restrict__ V = f.V;
+  const T* __restrict__ A = f.A;
+  const T* __restrict__ B = f.B;
+  T* __restrict__ Gb = f.Gb;
+  T* __restrict__ GBb = f.GBb;
   const int64_t id = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (id >= (int64_t)D.d[0] * D.d[1] * D.d[2]) return;
   int i, j, k;
@@ -464,40 +493,60 @@ int adj_step_t(fs_ctx* c, AdjStep& t, AdjWork& w, double grav[3]) {
   FS_HIP(c, hipGetLastError());
   // 7-8. extrapolation masks; gravity; extrapolation reversed (A: current array, B: buffer)
   const int iters = c->cfg.vel_extrapolate_iters;
+  int nbk[3], part0[4] = {0, 0, 0, 0};  // blocks of a face grid, and its first entry of the partial sums
   for (int a = 0; a < 3; a++) {
-    const int64_t nf = c->n_face[a];
-    Dims D = dims_of(c, a);
     while ((int)w.masks[a].size() < iters + 1) {
       w.masks[a].emplace_back();
-      FS_TRY(fs_alloc(c, w.masks[a].back(), (size_t)nf));
+      FS_TRY(fs_alloc(c, w.masks[a].back(), (size_t)c->n_face[a]));
     }
     FS_TRY(copy_buf(c, w.masks[a][0], t.valid[a]));
-    for (int it = 0; it < iters; it++)
-      k_extrap_mask<<<blocks(nf), TPB, 0, c->stream>>>(D, w.masks[a][it].as<uint8_t>(), w.masks[a][it + 1].as<uint8_t>());
-    const int nbk = blocks(nf);
-    if (w.part.bytes < (size_t)nbk * sizeof(double)) {
-      fs_free(w.part);
-      FS_TRY(fs_alloc(c, w.part, (size_t)nbk * sizeof(double)));
-    }
-    k_force_adj<T><<<nbk, TPB, 0, c->stream>>>(a, D, w.masks[a][iters].as<uint8_t>(), w.gb5[a].as<T>(),
-                                               w.part.as<double>());
-    std::vector<double> part(nbk);
-    FS_HIP(c, hipMemcpyAsync(part.data(), w.part.p, nbk * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    FS_HIP(c, hipStreamSynchronize(c->stream));
+    nbk[a] = blocks(c->n_face[a]);
+    part0[a + 1] = part0[a] + nbk[a];
+  }
+  const dim3 all(std::max(nbk[0], std::max(nbk[1], nbk[2])), 3);  // every face grid in one launch
+  for (int it = 0; it < iters; it++) {
+    MaskPass3 M;
+    for (int a = 0; a < 3; a++)
+      M.f[a] = {dims_of(c, a), w.masks[a][it].as<uint8_t>(), w.masks[a][it + 1].as<uint8_t>()};
+    k_extrap_mask<<<all, TPB, 0, c->stream>>>(M);
+  }
+  if (w.part.bytes < (size_t)part0[3] * sizeof(double)) {
+    fs_free(w.part);
+    FS_TRY(fs_alloc(c, w.part, (size_t)part0[3] * sizeof(double)));
+  }
+  for (int a = 0; a < 3; a++)
+    k_force_adj<T><<<nbk[a], TPB, 0, c->stream>>>(a, dims_of(c, a), w.masks[a][iters].as<uint8_t>(), w.gb5[a].as<T>(),
+                                                  w.part.as<double>() + part0[a]);
+  std::vector<double> part(part0[3]);
+  FS_HIP(c, hipMemcpyAsync(part.data(), w.part.p, part0[3] * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  FS_HIP(c, hipStreamSynchronize(c->stream));
+  DBuf *A[3], *B[3], *A2[3], *B2[3];
+  for (int a = 0; a < 3; a++) {
     double s = 0.0;
-    for (double v : part) s += v;
+    for (int q = part0[a]; q < part0[a + 1]; q++) s += part[q];
     grav[a] += dt * s;
-    DBuf *A = &w.gb5[a], *B = &w.B[a], *A2 = &w.A2[a], *B2 = &w.B2[a];
-    FS_HIP(c, hipMemsetAsync(B->p, 0, nf * R, c->stream));
-    for (int it = iters - 1; it >= 0; it--) {
-      k_extrap_adj<T><<<blocks(nf), TPB, 0, c->stream>>>(D, w.masks[a][it].as<uint8_t>(), A->as<T>(), B->as<T>(),
-                                                         A2->as<T>(), B2->as<T>());
-      std::swap(A, A2);
-      std::swap(B, B2);
+    A[a] = &w.gb5[a];
+    B[a] = &w.B[a];
+    A2[a] = &w.A2[a];
+    B2[a] = &w.B2[a];
+    FS_HIP(c, hipMemsetAsync(B[a]->p, 0, (size_t)c->n_face[a] * R, c->stream));
+  }
+  for (int it = iters - 1; it >= 0; it--) {
+    ExtrapAdj3<T> X;
+    for (int a = 0; a < 3; a++) {
+      X.f[a] = {dims_of(c, a),  w.masks[a][it].as<uint8_t>(), A[a]->as<T>(), B[a]->as<T>(),
+                A2[a]->as<T>(), B2[a]->as<T>()};
+      std::swap(A[a], A2[a]);
+      std::swap(B[a], B2[a]);
     }
+    k_extrap_adj<T><<<all, TPB, 0, c->stream>>>(X);
+  }
+  for (int a = 0; a < 3; a++) {
+    const int64_t nf = c->n_face[a];
+    const Dims D = dims_of(c, a);
     // 9. Dirichlet walls, plus FLIP's u_last; 10. P2G node fields
-    k_zero_walls<T><<<blocks(nf), TPB, 0, c->stream>>>(a, D, A->as<T>());
-    k_add<T><<<blocks(nf), TPB, 0, c->stream>>>(nf, A->as<T>(), w.gb0[a].as<T>());
+    k_zero_walls<T><<<blocks(nf), TPB, 0, c->stream>>>(a, D, A[a]->as<T>());
+    k_add<T><<<blocks(nf), TPB, 0, c->stream>>>(nf, A[a]->as<T>(), w.gb0[a].as<T>());
     k_p2g_fields<T><<<blocks(nf), TPB, 0, c->stream>>>(nf, w.gb0[a].as<T>(), t.w0[a].as<T>(), t.g0[a].as<T>(),
                                                        w.H[a].as<T>(), w.HG[a].as<T>());
     FS_HIP(c, hipGetLastError());

@@ -134,6 +134,25 @@ struct Grids3 {
   int d[3][3];
 };
 
+// The three face grids of a stage that treats them alike: one launch, the axis in blockIdx.y, blocks
+// enough in x for the largest grid. A launch of a few us per face grid, one after another, leaves a
+// small grid's stage waiting on launches (FP64, us, three launches / one: an extrapolation pass 14.3 /
+// 6.2 at 64^3, 30.1 / 21.9 at 128^3; wall faces 14.3 / 4.8 and 16.5 / 13.7; weights 22.7 / 13.7 and 76 /
+// 72; projection 12.7 / 5.8 and 30 / 25; collider 13.7 / 8.8 and 56 / 50; at 256^3 mixed both take the
+// same). The block's entry is read by its index: chosen by a ?: over the entries, the argument block
+// becomes a scratch array (5 to 15 times the kernel's time).
+template <typename T>
+struct Face {
+  int x, y, z;  // dimensions
+  T* g;         // velocity
+  T* w;         // weights, or the buffer of the velocity
+  uint8_t* valid;
+  uint8_t* vbuf;
+};
+template <typename T>
+struct Faces3 {
+  Face<T> f[3];
+};
 // sampleVelocity over the three face grids.
 template <typename T>
 __device__ inline V3<T> sample_velocity(const GridArgs<T>& ga, const Grids3<T>& G, T px, T py, T pz) {
@@ -1350,7 +1369,12 @@ __global__ __launch_bounds__(TPB) void k_smooth4(int nx, int ny, int nz, const T
 
 // applyDirichletBoundary (fluid-simulator.cc:113-138) for face grid `axis`.
 template <typename T>
-__global__ __launch_bounds__(TPB) void k_dirichlet(int axis, int gx, int gy, int gz, T* __restrict__ G, uint8_t* __restrict__ valid) {
+__global__ __launch_bounds__(TPB) void k_dirichlet(Faces3<T> F) {
+  const int axis = blockIdx.y;
+  const Face<T> f = F.f[axis];
+  const int gx = f.x, gy = f.y, gz = f.z;
+  T* __restrict__ G = f.g;
+  uint8_t* __restrict__ valid = f.valid;
   int id = blockIdx.x * blockDim.x + threadIdx.x;
   if (id >= gx * gy * gz) return;
   int i, j, k;
@@ -1365,10 +1389,11 @@ __global__ __launch_bounds__(TPB) void k_dirichlet(int axis, int gx, int gy, int
 
 // extrapolate<GridType> iteration (cpu/fluid-simulator.h:209-251).
 template <typename T>
-__global__ __launch_bounds__(TPB) void k_extrap_vel(int gx, int gy, int gz, const T* __restrict__ g, T* __restrict__ gbuf,
-                             const uint8_t* __restrict__ val, uint8_t* __restrict__ vbuf) {
-  int i, j, k, id;
-  if (!g3_index(gy, gz, i, j, k, id)) return;
+__device__ __forceinline__ void extrap_vel1(int id, int gx, int gy, int gz, const T* __restrict__ g,
+                                            T* __restrict__ gbuf, const uint8_t* __restrict__ val,
+                                            uint8_t* __restrict__ vbuf) {
+  int i, j, k;
+  unlin3(id, gy, gz, i, j, k);
   if (val[id]) {
     vbuf[id] = 1;
     return;
@@ -1396,17 +1421,13 @@ __global__ __launch_bounds__(TPB) void k_extrap_vel(int gx, int gy, int gz, cons
 // as one 4-byte load per direction, the values as four loads per direction where a flag asks for
 // them. Every face sums its valid neighbours in the order above and divides as above; valid faces
 // write only their flag (the value buffer keeps its stale entry). Other grids take
-// k_extrap_vel4f below (a byte-by-byte form of this kernel for them ran slower than the one-face
-// kernel).
+// extrap_vel4f below (a byte-by-byte form of this one for them ran slower than the one-face form).
 template <typename T>
-__global__ __launch_bounds__(TPB) void k_extrap_vel4(int gx, int gy, int gz, const T* __restrict__ g,
-                                                     T* __restrict__ gbuf, const uint8_t* __restrict__ val,
-                                                     uint8_t* __restrict__ vbuf) {
-  const int k0 = 4 * ((int)blockIdx.x * G3X + (int)threadIdx.x);
-  const int j = (int)blockIdx.y * G3Y + (int)threadIdx.y;
-  const int i = (int)blockIdx.z;
-  if (k0 >= gz || j >= gy) return;
-  const int id0 = (i * gy + j) * gz + k0;
+__device__ __forceinline__ void extrap_vel4(int id0, int gx, int gy, int gz, const T* __restrict__ g,
+                                            T* __restrict__ gbuf, const uint8_t* __restrict__ val,
+                                            uint8_t* __restrict__ vbuf) {
+  int i, j, k0;
+  unlin3(id0, gy, gz, i, j, k0);
   const int sx = gy * gz, sy = gz;
   auto flags = [&](int id) {
     const uchar4 f = *reinterpret_cast<const uchar4*>(val + id);
@@ -1467,12 +1488,10 @@ __global__ __launch_bounds__(TPB) void k_extrap_vel4(int gx, int gy, int gz, con
 // into place; each face masks every neighbour that is not on the grid (row and slab ends), so it
 // sums the same neighbours in the same order as the one-face kernel and writes what it writes.
 template <typename T>
-__global__ __launch_bounds__(TPB) void k_extrap_vel4f(int gx, int gy, int gz, const T* __restrict__ g,
-                                                      T* __restrict__ gbuf, const uint8_t* __restrict__ val,
-                                                      uint8_t* __restrict__ vbuf) {
+__device__ __forceinline__ void extrap_vel4f(int e0, int gx, int gy, int gz, const T* __restrict__ g,
+                                             T* __restrict__ gbuf, const uint8_t* __restrict__ val,
+                                             uint8_t* __restrict__ vbuf) {
   const int n = gx * gy * gz, sx = gy * gz, sy = gz;
-  const int e0 = 4 * (int)(blockIdx.x * TPB + threadIdx.x);
-  if (e0 >= n) return;
   auto word = [&](int p) { return *reinterpret_cast<const unsigned*>(val + p); };
   // flag bytes p .. p+3 (n is a multiple of 4: both words lie below n when p + 4 <= n)
   auto flags = [&](int p) -> unsigned {
@@ -1569,6 +1588,30 @@ __global__ __launch_bounds__(TPB) void k_extrap_vel4f(int gx, int gy, int gz, co
   *reinterpret_cast<unsigned*>(vbuf + e0) = fo;
 }
 
+// One pass over the three face grids: g and valid into w (the value buffer) and vbuf, four faces per
+// thread. The form follows from the grid's dimensions, alike for a block.
+template <typename T>
+__global__ __launch_bounds__(TPB) void k_extrap_vel(Faces3<T> F) {
+  const int a = blockIdx.y;
+  const Face<T> f = F.f[a];
+  const int gx = f.x, gy = f.y, gz = f.z;
+  const T* __restrict__ g = f.g;
+  T* __restrict__ gbuf = f.w;
+  const uint8_t* __restrict__ val = f.valid;
+  uint8_t* __restrict__ vbuf = f.vbuf;
+  const int n = gx * gy * gz, e0 = 4 * (int)(blockIdx.x * TPB + threadIdx.x);
+  if (gz % 4 == 0) {
+    if (e0 < n) extrap_vel4<T>(e0, gx, gy, gz, g, gbuf, val, vbuf);
+  } else if (gz >= 4 && (gy * gz) % 4 == 0) {
+    if (e0 < n) extrap_vel4f<T>(e0, gx, gy, gz, g, gbuf, val, vbuf);
+  } else {
+    for (int q = 0; q < 4; q++) {
+      const int id = (int)(blockIdx.x * 4 + q) * TPB + (int)threadIdx.x;
+      if (id < n) extrap_vel1<T>(id, gx, gy, gz, g, gbuf, val, vbuf);
+    }
+  }
+}
+
 // applyForce (fluid-simulator.cc:13-18)
 template <typename T>
 __global__ __launch_bounds__(TPB) void k_force(int gx, int gy, int gz, T* __restrict__ V, const uint8_t* __restrict__ valid, T gdt) {
@@ -1582,8 +1625,12 @@ __global__ __launch_bounds__(TPB) void k_force(int gx, int gy, int gz, T* __rest
 // Face solid weights of FvmSolver3D::buildSystem (project-solver.cc:77-127): faces between
 // two air cells keep 0; otherwise 1 - fractionInside of the collider SDF at the 4 corners.
 template <typename T>
-__global__ __launch_bounds__(TPB) void k_face_weights(int axis, GridArgs<T> ga, int gx, int gy, int gz, const T* __restrict__ fs,
-                               const T* __restrict__ col, T* __restrict__ W) {
+__global__ __launch_bounds__(TPB) void k_face_weights(Faces3<T> F, GridArgs<T> ga, const T* __restrict__ fs,
+                                const T* __restrict__ col) {
+  const int axis = blockIdx.y;
+  const Face<T> f = F.f[axis];
+  const int gx = f.x, gy = f.y, gz = f.z;
+  T* __restrict__ W = f.w;
   int id = blockIdx.x * blockDim.x + threadIdx.x;
   if (id >= gx * gy * gz) return;
   int i, j, k;
@@ -1730,8 +1777,13 @@ __global__ __launch_bounds__(TPB) void k_assemble(GridArgs<T> ga, T dt, const T*
 
 // FvmSolver3D::project (project-solver.cc:348-421) for face grid `axis`.
 template <typename T>
-__global__ __launch_bounds__(TPB) void k_project(int axis, GridArgs<T> ga, int gx, int gy, int gz, T dt, const T* __restrict__ fs,
-                          const T* __restrict__ pg, const T* __restrict__ Wt, T* __restrict__ G) {
+__global__ __launch_bounds__(TPB) void k_project(Faces3<T> F, GridArgs<T> ga, T dt, const T* __restrict__ fs,
+                          const T* __restrict__ pg) {
+  const int axis = blockIdx.y;
+  const Face<T> f = F.f[axis];
+  const int gx = f.x, gy = f.y, gz = f.z;
+  const T* __restrict__ Wt = f.w;
+  T* __restrict__ G = f.g;
   int id = blockIdx.x * blockDim.x + threadIdx.x;
   if (id >= gx * gy * gz) return;
   if (Wt[id] <= T(0)) return;
@@ -1764,8 +1816,11 @@ __global__ __launch_bounds__(TPB) void k_project(int axis, GridArgs<T> ga, int g
 
 // applyCollider (fluid-simulator.cc:76-111) for face grid `axis`.
 template <typename T>
-__global__ __launch_bounds__(TPB) void k_collider(int axis, GridArgs<T> ga, int gx, int gy, int gz, const T* __restrict__ col,
-                           T* __restrict__ G) {
+__global__ __launch_bounds__(TPB) void k_collider(Faces3<T> F, GridArgs<T> ga, const T* __restrict__ col) {
+  const int axis = blockIdx.y;
+  const Face<T> f = F.f[axis];
+  const int gx = f.x, gy = f.y, gz = f.z;
+  T* __restrict__ G = f.g;
   int id = blockIdx.x * blockDim.x + threadIdx.x;
   if (id >= gx * gy * gz) return;
   int i, j, k;
@@ -2162,32 +2217,37 @@ int p2g_t(fs_ctx* c) {
   return p2g_run<T, P2G_NORM>(c, c->pos, c->vel, !timed, batch, set);
 }
 
+// the face grids with their weights (w: of the context, or another array) and flags, and the launch
+// shape of n threads for every `per` faces
+template <typename T>
+Faces3<T> faces3(const fs_ctx* c, const DBuf* w) {
+  Faces3<T> F;
+  for (int a = 0; a < 3; a++)
+    F.f[a] = {c->fdim[a][0],  c->fdim[a][1], c->fdim[a][2], c->g[a].as<T>(), w[a].as<T>(), c->gvalid[a].as<uint8_t>(),
+              c->gvalidbuf[a].as<uint8_t>()};
+  return F;
+}
+dim3 faces3_grid(const fs_ctx* c, int per) {
+  const int64_t n = std::max(c->n_face[0], std::max(c->n_face[1], c->n_face[2]));
+  return dim3(fs_blocks((n + per - 1) / per, TPB), 3);
+}
+
 template <typename T>
 int dirichlet_t(fs_ctx* c) {
-  for (int a = 0; a < 3; a++)
-    k_dirichlet<T><<<fs_blocks(c->n_face[a], TPB), TPB, 0, c->stream>>>(a, c->fdim[a][0], c->fdim[a][1], c->fdim[a][2],
-                                                                        c->g[a].as<T>(), c->gvalid[a].as<uint8_t>());
+  k_dirichlet<T><<<faces3_grid(c, 1), TPB, 0, c->stream>>>(faces3<T>(c, c->gweights));
   FS_HIP(c, hipGetLastError());
   return FS_OK;
 }
 
 template <typename T>
 int extrap_vel_t(fs_ctx* c, int iters) {
-  for (int a = 0; a < 3; a++)
-    for (int it = 0; it < iters; it++) {
-      const int gx = c->fdim[a][0], gy = c->fdim[a][1], gz = c->fdim[a][2];
-      if (gz % 4 == 0)
-        k_extrap_vel4<T><<<g3_grid(gx, gy, gz / 4), g3_block(), 0, c->stream>>>(
-            gx, gy, gz, c->g[a].as<T>(), c->gbuf[a].as<T>(), c->gvalid[a].as<uint8_t>(), c->gvalidbuf[a].as<uint8_t>());
-      else if (gz >= 4 && (gy * gz) % 4 == 0)
-        k_extrap_vel4f<T><<<fs_blocks(c->n_face[a] / 4, TPB), TPB, 0, c->stream>>>(
-            gx, gy, gz, c->g[a].as<T>(), c->gbuf[a].as<T>(), c->gvalid[a].as<uint8_t>(), c->gvalidbuf[a].as<uint8_t>());
-      else
-        k_extrap_vel<T><<<g3_grid(gx, gy, gz), g3_block(), 0, c->stream>>>(
-            gx, gy, gz, c->g[a].as<T>(), c->gbuf[a].as<T>(), c->gvalid[a].as<uint8_t>(), c->gvalidbuf[a].as<uint8_t>());
+  for (int it = 0; it < iters; it++) {
+    k_extrap_vel<T><<<faces3_grid(c, 4), TPB, 0, c->stream>>>(faces3<T>(c, c->gbuf));
+    for (int a = 0; a < 3; a++) {
       std::swap(c->g[a], c->gbuf[a]);
       std::swap(c->gvalid[a], c->gvalidbuf[a]);
     }
+  }
   FS_HIP(c, hipGetLastError());
   return FS_OK;
 }
@@ -2204,10 +2264,8 @@ int force_t(fs_ctx* c, double dt) {
 template <typename T>
 int build_t(fs_ctx* c, double dt) {
   GridArgs<T> ga = grid_args<T>(c);
-  for (int a = 0; a < 3; a++)
-    k_face_weights<T><<<fs_blocks(c->n_face[a], TPB), TPB, 0, c->stream>>>(
-        a, ga, c->fdim[a][0], c->fdim[a][1], c->fdim[a][2], c->fsdf.as<T>(), c->collider.as<T>(),
-        c->gweights[a].as<T>());
+  k_face_weights<T><<<faces3_grid(c, 1), TPB, 0, c->stream>>>(faces3<T>(c, c->gweights), ga, c->fsdf.as<T>(),
+                                                              c->collider.as<T>());
   // Aneighbour order Left, Right, Up, Down, Front, Back (project-solver.cc:7-14)
   k_assemble<T><<<fs_blocks(c->n_cell, TPB), TPB, 0, c->stream>>>(
       ga, (T)dt, c->fsdf.as<T>(), c->gweights[0].as<T>(), c->gweights[1].as<T>(), c->gweights[2].as<T>(),
@@ -2222,11 +2280,8 @@ int build_t(fs_ctx* c, double dt) {
 template <typename T>
 int project_t(fs_ctx* c, double dt) {
   GridArgs<T> ga = grid_args<T>(c);
-  for (int a = 0; a < 3; a++)
-    k_project<T><<<fs_blocks(c->n_face[a], TPB), TPB, 0, c->stream>>>(a, ga, c->fdim[a][0], c->fdim[a][1],
-                                                                      c->fdim[a][2], (T)dt, c->fsdf.as<T>(),
-                                                                      c->pg.as<T>(), c->gweights[a].as<T>(),
-                                                                      c->g[a].as<T>());
+  k_project<T><<<faces3_grid(c, 1), TPB, 0, c->stream>>>(faces3<T>(c, c->gweights), ga, (T)dt, c->fsdf.as<T>(),
+                                                         c->pg.as<T>());
   FS_HIP(c, hipGetLastError());
   return FS_OK;
 }
@@ -2234,10 +2289,7 @@ int project_t(fs_ctx* c, double dt) {
 template <typename T>
 int collider_t(fs_ctx* c) {
   GridArgs<T> ga = grid_args<T>(c);
-  for (int a = 0; a < 3; a++)
-    k_collider<T><<<fs_blocks(c->n_face[a], TPB), TPB, 0, c->stream>>>(a, ga, c->fdim[a][0], c->fdim[a][1],
-                                                                       c->fdim[a][2], c->collider.as<T>(),
-                                                                       c->g[a].as<T>());
+  k_collider<T><<<faces3_grid(c, 1), TPB, 0, c->stream>>>(faces3<T>(c, c->gweights), ga, c->collider.as<T>());
   FS_HIP(c, hipGetLastError());
   return FS_OK;
 }
