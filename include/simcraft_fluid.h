@@ -95,7 +95,8 @@ typedef struct fs_config {
                                      has dropped tenfold and whenever it claims convergence), not
                                      nested solves with an inner tolerance */
   int32_t max_refinements;        /* unused, kept for layout (see inner_tolerance) */
-  int32_t check_interval;         /* PCG iterations between host convergence reads */
+  int32_t check_interval;         /* PCG iterations between host convergence reads (multigrid: at most this many,
+                                     and at most 2, are queued beyond the last one the host has seen) */
   int32_t profile_stages;         /* 1 = record per-stage device times into fs_stats (the fluid-SDF
                                      stages then stay on the main stream, so ms_reconstruct is
                                      their time); 2 = also per-launch kernel timing (see

@@ -99,6 +99,9 @@ struct MgState {
   DBuf x, r, s0, s1, t;  // CG vectors (FP64); z is level 0's x
   DBuf partials, partials2, scal;
   PcgScalars* host_scal = nullptr;  // pinned
+  // How far a running solve has come: the last finished iteration, or'ed with MG_STOPPED once it has
+  // stopped. A word of pinned memory that the device writes while the host queues iterations.
+  int *prog = nullptr, *prog_dev = nullptr;  // as the host and as the device address it
   int nchunks = 0;
 };
 

@@ -418,6 +418,13 @@ __global__ __launch_bounds__(1024) void k_mg_tail(TailLevels<S> T, int l0, int n
   for (int c = tid; c < n0; c += 1024) T.x[c] = vx[c];
 }
 
+// Iteration iter of a solve is finished (the thread that has written its scalars).
+constexpr int MG_STOPPED = 1 << 30;
+__device__ inline void report(int* prog, int iter, const PcgScalars* sc) {
+  __hip_atomic_store(prog, iter | (sc->converged != STOP_RUN ? MG_STOPPED : 0), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ---- CG kernels ---------------------------------------------------------------------------------
 // r = rhs on active cells (0 elsewhere), x = 0; ||r||_inf, ||r||_2^2 and the stopping test at
 // iteration 0.
@@ -477,7 +484,7 @@ template <typename S, int TH>
 __global__ __launch_bounds__(TH) void k_mg_spmv(Lv<S> L, const uint8_t* __restrict__ act, const S* __restrict__ z,
                                                  const double* __restrict__ s_old, double* __restrict__ s_new,
                                                  double* __restrict__ t, double* __restrict__ part, int nchunks,
-                                                 PcgScalars* sc, int iter) {
+                                                 PcgScalars* sc, int iter, int* prog) {
   __shared__ double sm[4];
   if (sc->converged != STOP_RUN) return;
   const int64_t n = (int64_t)L.nx * L.ny * L.nz;
@@ -520,6 +527,7 @@ __global__ __launch_bounds__(TH) void k_mg_spmv(Lv<S> L, const uint8_t* __restri
         sc->converged = STOP_ABORT;
         sc->status = FS_BREAKDOWN;
         sc->conv_iter = iter;
+        report(prog, iter, sc);
       } else {
         sc->alpha = sc->sigma / sdott;
       }
@@ -534,7 +542,8 @@ __global__ __launch_bounds__(TH) void k_mg_update(int64_t n, const uint8_t* __re
                                                    double* __restrict__ x, const double* __restrict__ s,
                                                    double* __restrict__ r, const double* __restrict__ t,
                                                    double* __restrict__ part, double* __restrict__ part2,
-                                                   int nchunks, PcgScalars* sc, int iter, int tol_mode, double tol) {
+                                                   int nchunks, PcgScalars* sc, int iter, int tol_mode, double tol,
+                                                   int* prog) {
   __shared__ double sm[4];
   if (sc->converged != STOP_RUN) return;
   const double alpha = sc->alpha;
@@ -584,6 +593,7 @@ __global__ __launch_bounds__(TH) void k_mg_update(int64_t n, const uint8_t* __re
         sc->converged = STOP_CONVERGED;
         sc->conv_iter = iter;
       }
+      report(prog, iter, sc);
     }
   }
 }
@@ -759,8 +769,10 @@ int mg_vectors(fs_ctx* c) {
   if (!M.scal.p) {
     FS_TRY(fs_alloc(c, M.scal, sizeof(PcgScalars)));
     FS_HIP(c, hipMemsetAsync(M.scal.p, 0, sizeof(PcgScalars), c->stream));
-    FS_HIP(c, hipHostMalloc((void**)&M.host_scal, sizeof(PcgScalars), hipHostMallocDefault));
   }
+  if (!M.host_scal) FS_HIP(c, hipHostMalloc((void**)&M.host_scal, sizeof(PcgScalars), hipHostMallocDefault));
+  if (!M.prog) FS_HIP(c, hipHostMalloc((void**)&M.prog, sizeof(int), hipHostMallocMapped));
+  if (!M.prog_dev) FS_HIP(c, hipHostGetDevicePointer((void**)&M.prog_dev, M.prog, 0));
   if (M.nchunks < nc || !M.partials.p) {
     FS_TRY(ensure(c, M.partials, (size_t)nc * sizeof(double)));
     FS_TRY(ensure(c, M.partials2, (size_t)nc * sizeof(double)));
@@ -779,6 +791,34 @@ int mg_read_scalars(fs_ctx* c) {
   FS_HIP(c, hipStreamSynchronize(c->stream));
   return FS_OK;
 }
+
+// Waits until iteration iter is finished or the solve has stopped.
+int mg_wait(fs_ctx* c, int iter, bool* stopped) {
+  for (unsigned n = 1;; n++) {
+    bool idle = false;
+    if (n % 1024 == 0) {  // a failed device never reports
+      const hipError_t e = hipStreamQuery(c->stream);
+      (void)hipGetLastError();  // "not ready" is not an error
+      if (e != hipErrorNotReady) FS_HIP(c, e);
+      idle = e == hipSuccess;
+    }
+    const int v = __atomic_load_n(c->mg.prog, __ATOMIC_RELAXED);
+    *stopped = (v & MG_STOPPED) != 0;
+    if (*stopped || v >= iter) return FS_OK;
+    if (idle) {
+      c->set_error("multigrid CG: an iteration ended without reporting");
+      return FS_DEVICE_ERROR;
+    }
+    __builtin_ia32_pause();
+  }
+}
+
+// Iterations queued beyond the last one reported. An iteration takes 60 us or more and queueing its 8 to
+// 20 launches about half of that, so the device stays busy, and a solve that has stopped leaves two
+// iterations of launches behind that return at once. Reading the scalars after every eighth iteration
+// left up to seven, half of a solve of ten, and the device idle meanwhile (mixed, ms per pass: 64^3
+// frames 14.6 / 12.9, 48^3 rollout 92 / 81, 256^3 frames alike).
+constexpr int MG_AHEAD = 2;
 
 template <typename S>
 int mg_solve_t(fs_ctx* c, fs_stats* st) {
@@ -806,38 +846,45 @@ int mg_solve_t(fs_ctx* c, fs_stats* st) {
     const Lv<S> L = lv_of<S>(L0);
     FS_TRY(mg_cycle<S>(c, M.r.as<double>(), sc, true));
     const int maxit = c->cfg.cg_max_iterations;
-    const int chk = std::max(1, c->cfg.check_interval);
+    const int chk = std::max(1, c->cfg.check_interval), ahead = std::min(chk, MG_AHEAD);
+    const bool timed = c->cfg.profile_stages >= 2 && c->ktime_on;  // kernels are timed one by one
+    __atomic_store_n(M.prog, 0, __ATOMIC_RELAXED);  // nothing that writes it is queued
+    int* prog = M.prog_dev;
     DBuf* sb[2] = {&M.s0, &M.s1};
-    int it = 1;
     bool stopped = false;
-    while (it < maxit && !stopped) {
-      for (int m = 0; m < chk && it < maxit; m++, it++) {
-        const double* s_old = sb[(it + 1) & 1]->as<double>();
-        double* s_new = sb[it & 1]->as<double>();
-        int pf = fs_prof_begin(c, FS_KERNEL_SPMV, (24.0 + 5.0 * sizeof(S)) * c->n_active_last);
-        auto spmv = [&](auto kern, int th) {
-          kern<<<nb, th, 0, c->stream>>>(L, act, L0.x.as<S>(), s_old, s_new, M.t.as<double>(), M.partials.as<double>(),
-                                         nc, sc, it);
-        };
-        if (nb <= MG_WIDE) spmv(k_mg_spmv<S, 1024>, 1024);
-        else spmv(k_mg_spmv<S, 256>, 256);
-        fs_prof_end(c, pf);
-        pf = fs_prof_begin(c, FS_KERNEL_PCG_UPDATE, 48.0 * c->n_active_last);
-        auto update = [&](auto kern, int th) {
-          kern<<<nb, th, 0, c->stream>>>(n, act, M.x.as<double>(), s_new, M.r.as<double>(), M.t.as<double>(),
-                                         M.partials.as<double>(), M.partials2.as<double>(), nc, sc, it, tmode, tol);
-        };
-        if (nb <= MG_WIDE) update(k_mg_update<1024>, 1024);
-        else update(k_mg_update<256>, 256);
-        fs_prof_end(c, pf);
-        FS_TRY(mg_cycle<S>(c, M.r.as<double>(), sc, false));
+    for (int it = 1; it < maxit && !stopped; it++) {
+      if (!timed) {
+        if (it > ahead) FS_TRY(mg_wait(c, it - ahead, &stopped));
+        if (stopped) break;
       }
+      const double* s_old = sb[(it + 1) & 1]->as<double>();
+      double* s_new = sb[it & 1]->as<double>();
+      int pf = fs_prof_begin(c, FS_KERNEL_SPMV, (24.0 + 5.0 * sizeof(S)) * c->n_active_last);
+      auto spmv = [&](auto kern, int th) {
+        kern<<<nb, th, 0, c->stream>>>(L, act, L0.x.as<S>(), s_old, s_new, M.t.as<double>(), M.partials.as<double>(),
+                                       nc, sc, it, prog);
+      };
+      if (nb <= MG_WIDE) spmv(k_mg_spmv<S, 1024>, 1024);
+      else spmv(k_mg_spmv<S, 256>, 256);
+      fs_prof_end(c, pf);
+      pf = fs_prof_begin(c, FS_KERNEL_PCG_UPDATE, 48.0 * c->n_active_last);
+      auto update = [&](auto kern, int th) {
+        kern<<<nb, th, 0, c->stream>>>(n, act, M.x.as<double>(), s_new, M.r.as<double>(), M.t.as<double>(),
+                                       M.partials.as<double>(), M.partials2.as<double>(), nc, sc, it, tmode, tol,
+                                       prog);
+      };
+      if (nb <= MG_WIDE) update(k_mg_update<1024>, 1024);
+      else update(k_mg_update<256>, 256);
+      fs_prof_end(c, pf);
+      FS_TRY(mg_cycle<S>(c, M.r.as<double>(), sc, false));
       FS_HIP(c, hipGetLastError());
-      FS_TRY(mg_read_scalars(c));
-      fs_prof_flush(c);
-      if (hs->wait_timeouts != 0) break;
-      if (hs->converged != STOP_RUN) stopped = true;
+      if (timed && (it % chk == 0 || it + 1 == maxit)) {
+        FS_TRY(mg_read_scalars(c));
+        fs_prof_flush(c);
+        stopped = hs->wait_timeouts != 0 || hs->converged != STOP_RUN;
+      }
     }
+    FS_TRY(mg_read_scalars(c));
     if (hs->wait_timeouts != 0) {
       c->set_error("multigrid CG: a reduction wait exceeded its bound");
       return FS_DEVICE_ERROR;
@@ -897,5 +944,7 @@ void fs_mg_release(fs_ctx* c) {
   for (DBuf* d : {&M.x, &M.r, &M.s0, &M.s1, &M.t, &M.partials, &M.partials2, &M.scal}) fs_free(*d);
   if (M.host_scal) (void)hipHostFree(M.host_scal);
   M.host_scal = nullptr;
+  if (M.prog) (void)hipHostFree(M.prog);
+  M.prog = M.prog_dev = nullptr;
   M.nchunks = 0;
 }
