@@ -221,9 +221,10 @@ __global__ __launch_bounds__(256) void k_mg_pre(Lv<S> L, const B* __restrict__ b
 
 // CHILD: one thread per child, the aggregate's sum over eight lanes; else one thread per aggregate.
 // Eight residuals of seven operands each, one after another in a thread, are the slowest sweep of a
-// small level (mixed, us, an aggregate / a child per thread: 7.2 / 3.3 for 64^3 -> 32^3, 11.0 / 10.0
-// for 128^3); above, other waves hide them and the eightfold threads and their shuffles cost more
-// than they save (14.8 / 17.0 for 160^3, 39.8 / 54.5 for 256^3).
+// small level (mixed, us, an aggregate / a child per thread, with a branch per term of a row: 7.2 / 3.3
+// for 64^3 -> 32^3, 11.0 / 10.0 for 128^3); above, other waves hide them and the eightfold threads and
+// their shuffles cost more than they save (14.8 / 17.0 for 160^3, 39.8 / 54.5 for 256^3). The chosen
+// forms take 3.7, 9.9, 11.7 and 38.1 with selects.
 constexpr int64_t MG_RESTRICT_CHILD = (int64_t)1 << 18;  // aggregates up to which CHILD is taken
 template <typename S, typename B, bool CHILD>
 __global__ __launch_bounds__(256) void k_mg_restrict(Lv<S> L, const B* __restrict__ b, const S* __restrict__ x,
